@@ -32,6 +32,8 @@
 
 #include "nans_narrow.hpp"
 
+#include <type_traits>
+
 namespace nans {
 
 constexpr int EPA_MAXV = 72;   // 4 + 65 vertices at most (one per iteration)
@@ -694,16 +696,20 @@ __device__ inline EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, cons
 // so the result is always epa_wave's.
 constexpr int EPA_SPILL = 99;
 
+// A set of lanes, face positions or vertex classes of a G-lane group.
+template <int G>
+using GroupMask = std::conditional_t<(G > 32), unsigned long long, uint32_t>;
+
 template <int G>
 struct EpgLds {
     static_assert(G == 16 || G == 32, "groups of 16 or 32 lanes");
     float vp[64 / G][G][3];   // vertex P per group
-    float sf[64 / G][G][9];   // compaction staging: n, a, d, id, cl
-    int ekey[64];             // horizon edges per group (G each)
-    int eids[64];
-    // horizon: how often the visible faces push each directed edge (ca, cb),
-    // one byte per key ca * G + cb, four keys per word
-    uint32_t ecnt[64 / G][G * G / 4];
+    int edge[64];             // horizon edges per group (G each): ids a | b << 8, classes ca << 16 | cb << 24
+    // horizon: the directed edges (ca, cb) that the visible faces push, bit cb of
+    // word ca
+    GroupMask<G> pushed[64 / G][G];
+    GroupMask<G> seen[64 / G];      // positions of the visible faces
+    GroupMask<G> kept[64 / G][2];   // low and high bit of the number of edges each keeps, by position
 };
 static_assert(sizeof(EpgLds<16>) <= sizeof(EpaLds), "the grouped EPA reuses the wave's EPA LDS");
 static_assert(sizeof(EpgLds<32>) <= sizeof(EpaLds), "the grouped EPA reuses the wave's EPA LDS");
@@ -919,22 +925,28 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
         const int cc = c == 1 ? C1 : (c == 2 ? C2 : C3);
         if (j < 4) F = make_face(Pa, Pb, Pc, a, b, c, ca, cb, cc);
     }
-    int nf = 4, nv = 4, iter = 0;
+    // A face stays in the lane that made it; pos is its index in the reference's
+    // face vector.  Erasing keeps the vector's order and new faces follow in edge
+    // order, so a survivor's position falls by the visible faces before it, and the
+    // new faces take the free lanes: no face is moved (staging the survivors and the
+    // new faces through LDS and reading them back was 27 LDS accesses a trip; 1M
+    // random pairs 4.75 -> 4.55 ms, 200k in the islands mode 1.61 -> 1.57 ms).
+    bool al = j < 4;
+    int pos = j, nf = 4, nv = 4, iter = 0;
     // A group that converges keeps its closest face (and, for the islands choice,
-    // face 0's distance and the winner's index) and stops: its polytope is frozen
-    // from then on, so the contact points are computed once for every group
-    // after the loop rather than on each iteration where some group converges.
+    // that face's lane) and stops: its polytope is frozen from then on, so the
+    // contact points are computed once for every group after the loop rather than
+    // on each iteration where some group converges.
     bool cv = false;
     V3 cN = z;
-    float ccur = 0.0f, cd0 = 0.0f;
+    float ccur = 0.0f;
     int cfid = 0, cbest = 0;
-    // the horizon's edge counts (below), zero at the start of every trip
-    constexpr int CW = G * G / 4;  // words of counts per group, G / 4 per lane
-    auto clear_counts = [&]() {
-#pragma unroll
-        for (int k = 0; k < CW / G; ++k) L.ecnt[g][j * (CW / G) + k] = 0u;
+    // the horizon's sets (below), empty at the start of every trip
+    auto clear_sets = [&]() {
+        L.pushed[g][j] = 0u;
+        if (j < 3) (j == 0 ? L.seen[g] : L.kept[g][j - 1]) = 0u;
     };
-    clear_counts();
+    clear_sets();
     wave_sync();
     for (;;) {
         // while (iter++ <= MAX_EPA_ITERATIONS), per group
@@ -946,28 +958,37 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
             run = false;
         }
         if (!ballot(run)) break;
-        // closest face: the first face holding the minimum below face 0's distance
-        const float d0 = gbcast_f<G, 0>(gabs(dot(mk3(F.nx, F.ny, F.nz), mk3(F.ax, F.ay, F.az))));
-        const float k0 = (j < nf && F.d < d0) ? F.d : __builtin_inff();
+        // closest face: the first face (by position) holding the minimum below face
+        // 0's distance; F.d is also the scan's |dot(stored normal, A)|: the flip of
+        // the normal only negates the dot product
+        const uint32_t f0 = gbits(ballot(al && pos == 0));
+        const int first = f0 ? ffs64(f0) : 0;
+        const float d0 = gpull_f(F.d, gb + first);
+        const float k0 = (al && F.d < d0) ? F.d : __builtin_inff();
         const float m = group_min<G>(k0);
         const uint32_t b0 = gbits(ballot(k0 == m));
-        const int best = (m != __builtin_inff() && b0) ? ffs64(b0) : 0;
+        int best = (m != __builtin_inff() && b0) ? ffs64(b0) : first;
+        if (ballot(m != __builtin_inff() && (b0 & (b0 - 1u)))) {  // some group has a tie
+            const float kp = k0 == m ? (float)pos : (float)(2 * G);
+            const uint32_t bp = gbits(ballot(kp == group_min<G>(kp)));
+            if (m != __builtin_inff() && bp) best = ffs64(bp);
+        }
         const int owner = gb + best;
         const V3 N = mk3(gpull_f(F.nx, owner), gpull_f(F.ny, owner), gpull_f(F.nz, owner));
-        const float dsel = gpull_f(F.d, owner);
-        const float cur = m == __builtin_inff() ? d0 : dsel;
-        int fid = gpull_i(F.id, owner);
+        const float cur = m == __builtin_inff() ? d0 : m;
         // new support along the stored normal
         const Vtx ns = group_support<G>(sh, N);
         const bool conv = run && dot(N, ns.P) - cur < p.epa_tolerance;
-        if (conv) {
-            cv = true;
-            cN = N;
-            ccur = cur;
-            cd0 = d0;
-            cfid = fid;
-            cbest = best;
-            run = false;
+        if (ballot(conv)) {
+            const int fid = gpull_i(F.id, owner);
+            if (conv) {
+                cv = true;
+                cN = N;
+                ccur = gpull_f(F.d, owner);
+                cfid = fid;
+                cbest = best;
+                run = false;
+            }
         }
         if (run && nv >= G) {
             r.status = EPA_SPILL;
@@ -988,118 +1009,74 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
             r.nverts = nv;
         }
         // visibility
-        const bool w0 = run && j < nf && dot(mk3(F.nx, F.ny, F.nz), sub(ns.P, mk3(F.ax, F.ay, F.az))) > 0.0f;
-        const uint32_t vis = gbits(ballot(w0));
-        const int nvis = __popc(vis);
+        const bool w0 = run && al && dot(mk3(F.nx, F.ny, F.nz), sub(ns.P, mk3(F.ax, F.ay, F.az))) > 0.0f;
         // horizon: edges of the visible faces in face order; an edge survives iff its
-        // reverse is not among them, when no key is pushed twice (else spill).  The
-        // visible faces' directed edges between non-NaN classes (< G) are counted
-        // per key (at most 3G pushes, so a byte never wraps); bits of this lane's
-        // three edges: same key pushed twice (s2), reverse key pushed (r1) and
-        // pushed twice (r2).  Edges with a NaN class never match, as vertex ==
-        // never holds for them.  The counts are zero here: cleared before the loop
-        // and after each trip's last read of them.
+        // reverse is not among them, when no key is pushed twice (else spill: a bit of
+        // pushed[] found set).  Edges with a NaN class (not < G) never match, as
+        // vertex == never holds for them, and enter no set.  The sets are empty here:
+        // cleared before the loop and after each trip's last read of them.
         const int cl = F.cl;
+        const GroupMask<G> one = 1;
+        bool dup = false;
         if (w0) {
+            atomicOr(&L.seen[g], one << pos);
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
                 const int ke = edge_key(cl, e);
                 const int ca = ke & 255, cb = ke >> 8;
-                if (ca < G && cb < G) {  // classes are < G, or CLS_NAN
-                    const int key = ca * G + cb;
-                    atomicAdd(&L.ecnt[g][key >> 2], 1u << (8 * (key & 3)));
-                }
+                if (ca < G && cb < G) dup |= (atomicOr(&L.pushed[g][ca], one << cb) >> cb) & 1u;
             }
         }
         wave_sync();
-        uint32_t s2 = 0, r1 = 0, r2 = 0;
+        int keep = 0;
         if (w0) {
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
                 const int ke = edge_key(cl, e);
                 const int ca = ke & 255, cb = ke >> 8;
-                if (ca < G && cb < G) {
-                    const int key = ca * G + cb, rkey = cb * G + ca;
-                    const uint32_t nk = (L.ecnt[g][key >> 2] >> (8 * (key & 3))) & 255u;
-                    const uint32_t nr = (L.ecnt[g][rkey >> 2] >> (8 * (rkey & 3))) & 255u;
-                    s2 |= (nk >= 2u ? 1u : 0u) << e;
-                    r1 |= (nr >= 1u ? 1u : 0u) << e;
-                    r2 |= (nr >= 2u ? 1u : 0u) << e;
-                }
+                const bool rev = ca < G && cb < G && ((L.pushed[g][cb] >> ca) & 1u);
+                keep |= rev ? 0 : 1 << e;
             }
+            const int cnt = __popc(keep);
+            if (cnt & 1) atomicOr(&L.kept[g][0], one << pos);
+            if (cnt & 2) atomicOr(&L.kept[g][1], one << pos);
         }
-        uint32_t nanbits = 0;
-#pragma unroll
-        for (int e = 0; e < 3; ++e) {
-            const int ke = edge_key(cl, e);
-            nanbits |= ((ke & 255) == CLS_NAN || (ke >> 8) == CLS_NAN) ? (1u << e) : 0u;
-        }
-        const bool dup = w0 && ((s2 | r2) & ~nanbits & 7u) != 0u;
-        const int keep = w0 ? (int)(~r1 & 7u) : 0;   // NaN edges never match: r1 has no NaN bits
-        const int cnt = __popc(keep);
-        const uint32_t lower = (1u << j) - 1u;
-        const uint32_t p0 = gbits(ballot(cnt & 1)), p1 = gbits(ballot(cnt & 2));
-        const int ne = __popc(p0) + 2 * __popc(p1);
-        if (run && (gbits(ballot(dup)) != 0u || ne > G)) {
+        wave_sync();
+        const GroupMask<G> seen = L.seen[g], kept0 = L.kept[g][0], kept1 = L.kept[g][1];
+        const GroupMask<G> before = (one << pos) - 1u;  // positions before this face's
+        const int ne = __popc(kept0) + 2 * __popc(kept1);
+        const int nsurv = nf - __popc(seen);
+        if (run && (gbits(ballot(dup)) != 0u || nsurv + ne > G)) {
             r.status = EPA_SPILL;
             run = false;
         }
         if (run && keep) {
-            int o = __popc(p0 & lower) + 2 * __popc(p1 & lower);
+            int o = gb + __popc(kept0 & before) + 2 * __popc(kept1 & before);
             const int id = F.id;
 #pragma unroll
             for (int e = 0; e < 3; ++e) {
-                if ((keep >> e) & 1) {
-                    L.eids[gb + o] = edge_key(id, e);
-                    L.ekey[gb + o] = edge_key(cl, e);
-                    ++o;
-                }
+                if ((keep >> e) & 1) L.edge[o++] = edge_key(id, e) | (edge_key(cl, e) << 16);
             }
         }
         wave_sync();
-        clear_counts();  // every read of the counts is behind the sync above
-        int ea = 0, eb = 0, eca = 0, ecb = 0;
-        if (run && j < ne) {
-            const int k2 = L.ekey[gb + j], i2 = L.eids[gb + j];
-            ea = i2 & 255;
-            eb = i2 >> 8;
-            eca = k2 & 255;
-            ecb = k2 >> 8;
-        }
-        // ordered removal of the visible faces, then the new ones, through LDS
-        const bool al = j < nf && !w0;
-        const uint32_t alive = gbits(ballot(al));
-        const int nsurv = __popc(alive);
-        if (run && nsurv + ne > G) {
-            r.status = EPA_SPILL;
-            run = false;
-        }
-        FaceR gn = FaceR{0, 0, 0, 0, 0, 0, 0, 0, 0};
-        if (run && j < ne) gn = make_face(ns.P, ld3(L.vp[g], ea), ld3(L.vp[g], eb), vnew, ea, eb, ncls, eca, ecb);
-        auto stage = [&](int at, const FaceR &f) {
-            float *d = L.sf[g][at];
-            d[0] = f.nx; d[1] = f.ny; d[2] = f.nz;
-            d[3] = f.ax; d[4] = f.ay; d[5] = f.az;
-            d[6] = f.d;
-            d[7] = __int_as_float(f.id);
-            d[8] = __int_as_float(f.cl);
-        };
+        clear_sets();  // every read of the sets is behind the sync above
+        // the visible faces leave, the survivors move up, and free lane number r of
+        // the group makes the face of edge r
         if (run) {
-            if (al) stage(__popc(alive & lower), F);
-            if (j < ne) stage(nsurv + j, gn);
+            al = al && !w0;
+            if (al) pos -= __popc(seen & before);
         }
-        wave_sync();
+        const uint32_t idle = gbits(ballot(!al));
+        const int rf = __popc(idle & ((1u << j) - 1u));
         if (run) {
-            const int nfn = nsurv + ne;
-            if (j < nfn) {
-                const float *d = L.sf[g][j];
-                F.nx = d[0]; F.ny = d[1]; F.nz = d[2];
-                F.ax = d[3]; F.ay = d[4]; F.az = d[5];
-                F.d = d[6];
-                F.id = __float_as_int(d[7]);
-                F.cl = __float_as_int(d[8]);
+            if (!al && rf < ne) {
+                const int ed = L.edge[gb + rf];
+                const int ea = ed & 255, eb = (ed >> 8) & 255, eca = (ed >> 16) & 255, ecb = (ed >> 24) & 255;
+                F = make_face(ns.P, ld3(L.vp[g], ea), ld3(L.vp[g], eb), vnew, ea, eb, ncls, eca, ecb);
+                al = true;
+                pos = nsurv + rf;
             }
-            nf = nfn;
+            nf = nsurv + ne;
             if (nf > r.max_faces) r.max_faces = nf;
         }
         wave_sync();
@@ -1113,21 +1090,24 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
             // the final face by binary64 plane distance: the first of the least
             // below face 0's, else face 0 (epa_wave's islands choice per group)
             wave_sync();
-            const double d64 = j < nf ? group_face_dist64(L.vp[g], F) : 0.0;
-            const double f0 = __shfl(d64, gb, 64);
-            bool v64 = cv && j < nf && d64 < f0;
+            const double d64 = al ? group_face_dist64(L.vp[g], F) : 0.0;
+            const uint32_t m0 = gbits(ballot(al && pos == 0));
+            const int first = m0 ? ffs64(m0) : 0;
+            const double f0 = __shfl(d64, gb + first, 64);
+            bool v64 = cv && al && d64 < f0;
             double bd = v64 ? d64 : 0.0;
-            int bi = v64 ? j : 0x7fffffff;
+            int bi = v64 ? pos : 0x7fffffff;
             group_argmin64<G>(v64, bd, bi);
-            const int sel = v64 ? bi : 0;
             depth = v64 ? bd : f0;
+            const uint32_t ms = gbits(ballot(al && pos == bi));
+            const int sel = v64 && ms ? ffs64(ms) : first;  // its lane
             const int so = gb + sel;
             const V3 Ns = mk3(gpull_f(F.nx, so), gpull_f(F.ny, so), gpull_f(F.nz, so));
             const float ds = gpull_f(F.d, so);
             const int fs = gpull_i(F.id, so);
             if (sel != cbest) {
                 Nc = Ns;
-                cc = sel == 0 ? cd0 : ds;
+                cc = ds;
                 fid = fs;
             }
         }
