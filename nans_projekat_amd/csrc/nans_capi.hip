@@ -2,6 +2,7 @@
 // C ABI declared in include/nans_gpu.h.
 #include "nans_common.hpp"
 
+#include <algorithm>
 #include <mutex>
 #include <new>
 
@@ -57,12 +58,14 @@ __device__ inline void write_pair(const NarrowOutDev &o, int64_t i, int64_t n, i
     if (o.depth) o.depth[i] = depth;
 }
 
-// Candidates of one workgroup: pairs [base, base + count) of the input arrays.
+// Candidates of one wave: pairs [base, base + count) of the input arrays.
 struct PairSrc {
     NarrowIn a, b;
     int64_t base, n;
     NarrowOutDev o;
     unsigned long long *overflow;
+    SimplexRec *simplex;
+    __device__ SimplexRec &sim(int c) const { return simplex[c]; }
     static constexpr bool kMemCorners = false;
     __device__ int key(int c) const { return c; }
     __device__ void shapes_ref(int key, Shape &A, Shape &B) const { shapes(key, A, B); }
@@ -83,25 +86,40 @@ struct PairSrc {
     }
 };
 
-// Pairs per workgroup of the narrowphase entry point, and the kernel's occupancy
-// floor: three waves per SIMD (168 VGPRs, a few spilled) and short ranges, so
-// that slow EPA ranges are spread over many workgroups; on 1M random pairs this
-// runs 5.1 ms against 6.8 ms at two waves per SIMD and 1024-pair ranges.
-constexpr int NP_RANGE = 256;
+// The narrowphase entry point: every wave takes a share of the pairs on its own
+// (narrow_wave), so a small call is spread over the whole chip and no wave waits
+// for the slowest pair of its workgroup.  With 256 pairs per workgroup, 777 pairs
+// ran on four workgroups as a chain of EPA passes (756 us a call, now 136), 30011
+// on 117 of the chip's 256 CUs (942 us, now 440); 1M pairs 4.70 -> 4.03 ms.
+// Shares of at most 32 pairs, so that the last ones end together (1M pairs at 16,
+// 32, 64: 4.10, 3.90, 3.96 ms; 200k in the islands mode 1.19, 1.24, 1.36 ms), and
+// of a quarter of a wave's part of a smaller call, down to one pair.  Three waves
+// per SIMD (168 VGPRs; two take 5.37 ms where three take 4.82, four spill).
+constexpr int NP_SHARE = 32;
+constexpr int NP_WAVES_PER_CU = 12;
 
 // ISL: the FP64-islands mode (grouped EPA tiers with a binary64 final face).
 template <bool ISL>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_narrowphase(
-    int64_t n, NarrowIn a, NarrowIn b, NarrowParams p, NarrowOutDev o, unsigned long long *overflow, int *qidx,
-    SimplexRec *qsim)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PER_CU / 4))) void k_narrowphase(
+    int64_t n, int share, NarrowIn a, NarrowIn b, NarrowParams p, NarrowOutDev o, unsigned long long *cnt, int *list,
+    SimplexRec *sim)
 {
     __shared__ EpaLds lds[4];
-    __shared__ NarrowShared sh;
-    const int64_t base = (int64_t)blockIdx.x * NP_RANGE;
-    const int count = (int)min((int64_t)NP_RANGE, n - base);
-    PairSrc src{a, b, base, n, o, overflow};
-    narrow_block<256, true, ISL>(src, count, p, lds, sh, qidx + base, qsim + base);
-    if (threadIdx.x == 0 && sh.stalled) atomicAdd(overflow, (unsigned long long)sh.stalled);
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    int found = 0;
+    for (;;) {
+        unsigned long long t = 0;
+        wave_sync();  // the wave meets on both sides of the claim
+        if (lane_id() == 0) t = atomicAdd(&cnt[1], 1ull);
+        wave_sync();
+        t = ((unsigned long long)__builtin_amdgcn_readfirstlane((int)(t >> 32)) << 32) |
+            (unsigned)__builtin_amdgcn_readfirstlane((int)t);
+        const int64_t base = (int64_t)t * share;
+        if (base >= n) break;
+        const int count = (int)min((int64_t)share, n - base);
+        PairSrc src{a, b, base, n, o, &cnt[0], sim + base};
+        narrow_wave<true, ISL>(src, count, p, lds[wv], list + base, found);
+    }
 }
 
 __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
@@ -298,17 +316,22 @@ static int narrow_launch(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, con
                          int64_t *n_overflow)
 {
     hipStream_t s = ctx->stream;
-    k_fill_u64<<<1, 64, 0, s>>>(cnt, 1, 0ull);
+    k_fill_u64<<<1, 64, 0, s>>>(cnt, 2, 0ull);  // the overflow count, and the next share
     NANS_HIP(hipGetLastError());
     if (n > 0) {
         NarrowIn ia{a->type, a->pos, a->quat, a->half};
         NarrowIn ib{b->type, b->pos, b->quat, b->half};
         NarrowOutDev o{out->gjk, out->contact, out->status, out->normal, out->point_a, out->point_b, out->depth};
-        unsigned grid = (unsigned)((n + NP_RANGE - 1) / NP_RANGE);
+        int cus = 0;
+        NANS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->p.device));
+        const int64_t waves = NP_WAVES_PER_CU * (int64_t)cus;
+        const int share = (int)std::min<int64_t>(NP_SHARE, std::max<int64_t>(1, n / (4 * waves)));
+        const unsigned grid = (unsigned)std::min<int64_t>((n + 4 * share - 1) / (4 * share), waves / 4);
+        const NarrowParams np = narrow_params(ctx->p);
         if (ctx->p.fp64_islands)
-            k_narrowphase<true><<<grid, 256, 0, s>>>(n, ia, ib, narrow_params(ctx->p), o, cnt, qidx, qsim);
+            k_narrowphase<true><<<grid, 256, 0, s>>>(n, share, ia, ib, np, o, cnt, qidx, qsim);
         else
-            k_narrowphase<false><<<grid, 256, 0, s>>>(n, ia, ib, narrow_params(ctx->p), o, cnt, qidx, qsim);
+            k_narrowphase<false><<<grid, 256, 0, s>>>(n, share, ia, ib, np, o, cnt, qidx, qsim);
         NANS_HIP(hipGetLastError());
     }
     unsigned long long ov = 0;

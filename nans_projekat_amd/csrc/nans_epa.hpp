@@ -32,8 +32,6 @@
 
 #include "nans_narrow.hpp"
 
-#include <type_traits>
-
 namespace nans {
 
 constexpr int EPA_MAXV = 72;   // 4 + 65 vertices at most (one per iteration)
@@ -241,7 +239,7 @@ __device__ inline Vtx wave_support(const EpaShapes &s, V3 d)
     return v;
 }
 
-// Position of the n-th set bit of m (n < popcount(m)).
+// Position of the n-th set bit of m (n < __popc(m)).
 __device__ __forceinline__ int nth_set_bit(uint64_t m, int n)
 {
     int pos = 0;
@@ -696,10 +694,6 @@ __device__ inline EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, cons
 // so the result is always epa_wave's.
 constexpr int EPA_SPILL = 99;
 
-// A set of lanes, face positions or vertex classes of a G-lane group.
-template <int G>
-using GroupMask = std::conditional_t<(G > 32), unsigned long long, uint32_t>;
-
 template <int G>
 struct EpgLds {
     static_assert(G == 16 || G == 32, "groups of 16 or 32 lanes");
@@ -707,9 +701,9 @@ struct EpgLds {
     int edge[64];             // horizon edges per group (G each): ids a | b << 8, classes ca << 16 | cb << 24
     // horizon: the directed edges (ca, cb) that the visible faces push, bit cb of
     // word ca
-    GroupMask<G> pushed[64 / G][G];
-    GroupMask<G> seen[64 / G];      // positions of the visible faces
-    GroupMask<G> kept[64 / G][2];   // low and high bit of the number of edges each keeps, by position
+    uint32_t pushed[64 / G][G];
+    uint32_t seen[64 / G];      // positions of the visible faces
+    uint32_t kept[64 / G][2];   // low and high bit of the number of edges each keeps, by position
 };
 static_assert(sizeof(EpgLds<16>) <= sizeof(EpaLds), "the grouped EPA reuses the wave's EPA LDS");
 static_assert(sizeof(EpgLds<32>) <= sizeof(EpaLds), "the grouped EPA reuses the wave's EPA LDS");
@@ -821,11 +815,14 @@ __device__ inline Vtx group_support(const EpaShapes &s, V3 d)
     const float ka = onb ? ko : key, kb = onb ? key : ko;
     const V3 ca = mk3(onb ? co.x : cw.x, onb ? co.y : cw.y, onb ? co.z : cw.z);
     const V3 cb = mk3(onb ? cw.x : co.x, onb ? cw.y : co.y, onb ? cw.z : co.z);
+    // a sphere's support along -d is c - r n with the n of +d (as in minkowski):
+    // one normalize serves both shapes and every group
+    const bool sa = s.kind_a != SHAPE_BOX, sb = s.kind_b != SHAPE_BOX;
+    V3 n = mk3(0.0f, 0.0f, 0.0f);
+    if (sa || sb) n = normalize(d);
     Vtx v;
-    v.A = s.kind_a == SHAPE_BOX ? (ka == -__builtin_inff() ? mk3(0.0f, 0.0f, 0.0f) : ca)
-                                : sphere_support(s.ca, s.ra, d);
-    v.B = s.kind_b == SHAPE_BOX ? (kb == -__builtin_inff() ? mk3(0.0f, 0.0f, 0.0f) : cb)
-                                : sphere_support(s.cb, s.rb, nd);
+    v.A = sa ? add(s.ca, mul(n, s.ra)) : (ka == -__builtin_inff() ? mk3(0.0f, 0.0f, 0.0f) : ca);
+    v.B = sb ? sub(s.cb, mul(n, s.rb)) : (kb == -__builtin_inff() ? mk3(0.0f, 0.0f, 0.0f) : cb);
     v.P = sub(v.A, v.B);
     return v;
 }
@@ -968,7 +965,7 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
         const float m = group_min<G>(k0);
         const uint32_t b0 = gbits(ballot(k0 == m));
         int best = (m != __builtin_inff() && b0) ? ffs64(b0) : first;
-        if (ballot(m != __builtin_inff() && (b0 & (b0 - 1u)))) {  // some group has a tie
+        if (ballot(m != __builtin_inff() && (b0 & (b0 - 1)))) {  // some group has a tie
             const float kp = k0 == m ? (float)pos : (float)(2 * G);
             const uint32_t bp = gbits(ballot(kp == group_min<G>(kp)));
             if (m != __builtin_inff() && bp) best = ffs64(bp);
@@ -1016,7 +1013,7 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
         // vertex == never holds for them, and enter no set.  The sets are empty here:
         // cleared before the loop and after each trip's last read of them.
         const int cl = F.cl;
-        const GroupMask<G> one = 1;
+        const uint32_t one = 1;
         bool dup = false;
         if (w0) {
             atomicOr(&L.seen[g], one << pos);
@@ -1042,11 +1039,11 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
             if (cnt & 2) atomicOr(&L.kept[g][1], one << pos);
         }
         wave_sync();
-        const GroupMask<G> seen = L.seen[g], kept0 = L.kept[g][0], kept1 = L.kept[g][1];
-        const GroupMask<G> before = (one << pos) - 1u;  // positions before this face's
+        const uint32_t seen = L.seen[g], kept0 = L.kept[g][0], kept1 = L.kept[g][1];
+        const uint32_t before = (one << pos) - 1;  // positions before this face's
         const int ne = __popc(kept0) + 2 * __popc(kept1);
         const int nsurv = nf - __popc(seen);
-        if (run && (gbits(ballot(dup)) != 0u || nsurv + ne > G)) {
+        if (run && (gbits(ballot(dup)) != 0 || nsurv + ne > G)) {
             r.status = EPA_SPILL;
             run = false;
         }
@@ -1067,7 +1064,7 @@ __device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0,
             if (al) pos -= __popc(seen & before);
         }
         const uint32_t idle = gbits(ballot(!al));
-        const int rf = __popc(idle & ((1u << j) - 1u));
+        const int rf = __popc(idle & ((one << j) - 1));
         if (run) {
             if (!al && rf < ne) {
                 const int ed = L.edge[gb + rf];
@@ -1281,12 +1278,10 @@ __device__ inline int gjk_lane_call(GjkLane &G, float *cyc, const NarrowParams &
 //   void shapes(int key, Shape &A, Shape &B) const       both shapes of the pair
 //   void gjk_result(int c, int gjk) const                 every candidate
 //   void epa_result(int c, int key, const EpaResult &r) const   every GJK hit (lane 0 calls)
-// WIDE: polytopes that outgrow a 16-lane group go to a 32-lane group before the
-// whole wave (worth its registers where many do, as among random deep overlaps).
 // ISL: the FP64-islands mode runs the grouped tiers too (their final face choice
 // in binary64); without it, that mode runs every polytope by the whole wave.
 // The team's wave k uses epa[k]; sh, qidx and qsim are the team's own.
-template <bool WIDE, bool ISL = false, class Src>
+template <bool ISL = false, class Src>
 __device__ void narrow_team(const Team &team, const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
                             NarrowShared &sh, int *qidx, SimplexRec *qsim)
 {
@@ -1338,12 +1333,9 @@ __device__ void narrow_team(const Team &team, const Src &src, int ncand, const N
     EpaLds &L = epa[team.rank >> 6];
     if (grouped) {
         // four pairs per wave, one per 16-lane group, started while other waves
-        // may still be in GJK; a spilled polytope is redone by the whole wave, or
-        // with WIDE by a 32-lane group (two at a time) and, if it spills there
-        // too, by the whole wave
+        // may still be in GJK; a spilled polytope is redone by the whole wave
         const int NW = team.waves();
         EpgLds<16> &G = *reinterpret_cast<EpgLds<16> *>(&L);
-        EpgLds<32> &G2 = *reinterpret_cast<EpgLds<32> *>(&L);
         const int j = lane & 15;
         // A pass takes four queue slots, one per group.  The next pass's slots are
         // claimed while this one starts, their contents loaded (relaxed) under its
@@ -1415,63 +1407,11 @@ __device__ void narrow_team(const Team &team, const Src &src, int ncand, const N
             wave_sync();
             const int nbase = claim();
             const int seen = peek(nbase);
-            // WIDE: a pair with a sphere goes to the 32-lane tier at once (a sphere's
-            // support gives a new vertex at every iteration, so its polytopes grow)
-            const bool sph = WIDE && (A.kind != SHAPE_BOX || B.kind != SHAPE_BOX);
-            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act && !sph, np);
-            if (act && !sph && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
-            const uint64_t spill = ballot(act && j == 0 && (sph || r.status == EPA_SPILL));
+            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np);
+            if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
+            const uint64_t spill = ballot(act && j == 0 && r.status == EPA_SPILL);
             wave_sync();
-            const int nsp = __popcll(spill);
-            for (int t = 0; WIDE && 2 * t < nsp; ++t) {
-                // spilled group k = 2t + h goes to 32-lane group h
-                const int h = lane >> 5, j2 = lane & 31;
-                const int k = 2 * t + h;
-                const bool act2 = k < nsp;
-                const int sg = nth_set_bit(spill, act2 ? k : 2 * t) >> 4;
-                const int cs = __shfl(c, 16 * sg, 64);
-                const int ks = __shfl(key, 16 * sg, 64);
-                const int sj = base + sg;
-                Shape SA, SB;
-                src.shapes(ks, SA, SB);
-                const EpaShapes e2 = epa_shapes_group(SA, SB);
-                V3 a2 = mk3(0.0f, 0.0f, 0.0f), b2 = a2;
-                if (j2 < 4) {
-                    const SimplexRec &q = qsim[sj];
-                    a2 = mk3(q.a[3 * j2], q.a[3 * j2 + 1], q.a[3 * j2 + 2]);
-                    b2 = mk3(q.b[3 * j2], q.b[3 * j2 + 1], q.b[3 * j2 + 2]);
-                }
-                wave_sync();
-                const EpaResult r2 = epa_group<32, ISL>(G2, e2, a2, b2, act2, np);
-                if (act2 && j2 == 0 && r2.status != EPA_SPILL) src.epa_result(cs, ks, r2);
-                uint64_t spill2 = ballot(act2 && j2 == 0 && r2.status == EPA_SPILL);
-                wave_sync();
-                while (spill2) {
-                    const int src_lane = ffs64(spill2);  // 0 or 32
-                    spill2 &= spill2 - 1;
-                    const int cw = __shfl(cs, src_lane, 64);
-                    const int kw = __shfl(ks, src_lane, 64);
-                    const int sw = __shfl(sj, src_lane, 64);
-                    Shape WA, WB;
-                    src.shapes(kw, WA, WB);
-                    const EpaShapes ew = epa_shapes(WA, WB);
-                    V3 p0 = mk3(0.0f, 0.0f, 0.0f);
-                    if (lane < 4) {
-                        const SimplexRec &q = qsim[sw];
-                        V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
-                        V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
-                        p0 = sub(a, b);
-                        st3(L.va, lane, a);
-                        st3(L.vb, lane, b);
-                        st3(L.vp, lane, p0);
-                    }
-                    wave_sync();
-                    const EpaResult rw = epa_wave(L, ew, p0, np);
-                    if (lane == 0) src.epa_result(cw, kw, rw);
-                    wave_sync();
-                }
-            }
-            for (uint64_t sp = WIDE ? 0ull : spill; sp; sp &= sp - 1) {
+            for (uint64_t sp = spill; sp; sp &= sp - 1) {
                 const int sg = ffs64(sp) >> 4;  // the spilled group
                 const int cs = __shfl(c, 16 * sg, 64);
                 const int ks = __shfl(key, 16 * sg, 64);
@@ -1529,12 +1469,175 @@ __device__ void narrow_team(const Team &team, const Src &src, int ncand, const N
     team.sync();
 }
 
+// EPA of one queued pair by the whole wave: supports of its four simplex vertices
+// in q, every lane returns the result.
+__device__ inline EpaResult epa_whole(EpaLds &L, const EpaShapes &es, const SimplexRec &q, const NarrowParams &np)
+{
+    const int lane = lane_id();
+    V3 p0 = mk3(0.0f, 0.0f, 0.0f);
+    if (lane < 4) {
+        const V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
+        const V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
+        p0 = sub(a, b);
+        st3(L.va, lane, a);
+        st3(L.vb, lane, b);
+        st3(L.vp, lane, p0);
+    }
+    wave_sync();
+    const EpaResult r = epa_wave(L, es, p0, np);
+    wave_sync();
+    return r;
+}
+
+// The same driver for one wave on its own: CheckCollision over the candidates
+// [0, ncand) of src, with no other wave to wait for.  A GJK hit's simplex goes to
+// sim(c), and the wave lists its hits in list[0, ncand): pairs for the narrow tier
+// from the front, pairs for the wide tier from the back.  The tiers then run over
+// dense lists: four pairs at a time in 16-lane groups, their spills with the wide
+// list two at a time in 32-lane groups (WIDE; else spills go to the whole wave),
+// and what outgrows those by the whole wave.  A wave with one hit gives it to the
+// whole wave at once, and two to the 32-lane tier, since the lanes are idle
+// otherwise and the narrow tiers' attempts would only lengthen the chain.
+template <bool WIDE, bool ISL, class Src>
+__device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list, int &found)
+{
+    const int lane = lane_id();
+    const uint64_t lower = (1ull << lane) - 1ull;
+    auto fence = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    int nn = 0, nw = 0;  // hits of the narrow and of the wide list
+    {
+        float *cyc = reinterpret_cast<float *>(&L);
+        GjkLane G;
+        int next = 0;
+        for (;;) {
+            const bool need = G.c < 0 && !G.retired;
+            const uint64_t m = ballot(need);
+            if (m && (__popcll(m) >= GJK_REFILL_MIN || !ballot(G.c >= 0))) {
+                if (need) gjk_lane_take(G, src, next + __popcll(m & lower), ncand, cyc);
+                next += __popcll(m);
+            }
+            if (!ballot(G.c >= 0)) break;
+            int g = GJK_STILL;
+            if (G.c >= 0) g = gjk_lane_call(G, cyc, np);
+            const bool hit = g == GJK_FOUND;
+            if (g != GJK_STILL) {
+                src.gjk_result(G.c, g);
+                if (hit) {
+                    SimplexRec &q = src.sim(G.c);
+                    simplex_rec_store(q, G.S);
+                    q.key = G.key;
+                }
+            }
+            // a sphere's support gives a new vertex at every iteration, so its polytopes
+            // outgrow a 16-lane group
+            const bool wide = WIDE && hit && (G.A.kind != SHAPE_BOX || G.B.kind != SHAPE_BOX);
+            const uint64_t mn = ballot(hit && !wide), mw = ballot(wide);
+            if (hit) list[wide ? ncand - 1 - nw - __popcll(mw & lower) : nn + __popcll(mn & lower)] = G.c;
+            nn += __popcll(mn);
+            nw += __popcll(mw);
+            if (g != GJK_STILL) G.c = -1;
+        }
+    }
+    found += nn + nw;
+    fence();
+    if (!ISL && np.fp64_islands) {  // the grouped tiers' islands choice is the ISL instantiation's
+        for (int k = 0; k < nn + nw; ++k) {
+            const int c = list[k < nn ? k : ncand - 1 - (k - nn)];
+            const SimplexRec &q = src.sim(c);
+            const int key = q.key;
+            Shape A, B;
+            src.shapes(key, A, B);
+            const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np);
+            if (lane == 0) src.epa_result(c, key, r);
+        }
+        fence();
+        return;
+    }
+    int nspill = 0;  // pairs that outgrew the narrow tier, at list[0, nspill)
+    if (nn + nw == 1) {
+        nspill = nn;
+    } else if (WIDE && nn + nw == 2) {
+        nspill = nn;
+    } else {
+        EpgLds<16> &G = *reinterpret_cast<EpgLds<16> *>(&L);
+        const int j = lane & 15;
+        for (int base = 0; base < nn; base += 4) {
+            const int k = base + (lane >> 4);
+            const bool act = k < nn;
+            const int c = list[act ? k : base];
+            const SimplexRec &q = src.sim(c);
+            const int key = q.key;
+            Shape A, B;
+            if constexpr (Src::kMemCorners) src.shapes_ref(key, A, B);
+            else src.shapes(key, A, B);
+            const EpaShapes es = epa_shapes_group<Src::kMemCorners>(A, B);
+            V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
+            if (j < 4) {
+                sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
+                sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
+            }
+            wave_sync();
+            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np);
+            if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
+            // the spilled pairs move to the front of the list, over entries already read
+            const bool sp = act && j == 0 && r.status == EPA_SPILL;
+            const uint64_t ms = ballot(sp);
+            if (sp) list[nspill + __popcll(ms & lower)] = c;
+            nspill += __popcll(ms);
+        }
+        fence();
+    }
+    // the wide tiers over the spills, then the wide list
+    const int nwide = nspill + nw;
+    auto item = [&](int k) { return list[k < nspill ? k : ncand - 1 - (k - nspill)]; };
+    auto whole = [&](int c) {
+        const SimplexRec &q = src.sim(c);
+        const int key = q.key;
+        Shape A, B;
+        src.shapes(key, A, B);
+        const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np);
+        if (lane == 0) src.epa_result(c, key, r);
+    };
+    if (!WIDE || nwide == 1) {
+        for (int k = 0; k < nwide; ++k) whole(item(k));
+    } else {
+        EpgLds<32> &G2 = *reinterpret_cast<EpgLds<32> *>(&L);
+        const int j = lane & 31;
+        for (int base = 0; base < nwide; base += 2) {
+            const int k = base + (lane >> 5);
+            const bool act = k < nwide;
+            const int c = item(act ? k : base);
+            const SimplexRec &q = src.sim(c);
+            const int key = q.key;
+            Shape A, B;
+            src.shapes(key, A, B);
+            const EpaShapes es = epa_shapes_group(A, B);
+            V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
+            if (j < 4) {
+                sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
+                sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
+            }
+            wave_sync();
+            const EpaResult r = epa_group<32, ISL>(G2, es, sa0, sb0, act, np);
+            if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
+            uint64_t sp = ballot(act && j == 0 && r.status == EPA_SPILL);
+            wave_sync();
+            for (; sp; sp &= sp - 1) whole(__builtin_amdgcn_readlane(c, ffs64(sp)));
+        }
+    }
+    fence();
+}
+
 // narrow_team by the whole workgroup of BLOCK threads
-template <int BLOCK, bool WIDE, bool ISL = false, class Src>
+template <int BLOCK, bool ISL = false, class Src>
 __device__ inline void narrow_block(const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
                                     NarrowShared &sh, int *qidx, SimplexRec *qsim)
 {
-    narrow_team<WIDE, ISL>(Team::block(BLOCK), src, ncand, np, epa, sh, qidx, qsim);
+    narrow_team<ISL>(Team::block(BLOCK), src, ncand, np, epa, sh, qidx, qsim);
 }
 
 }  // namespace nans

@@ -471,7 +471,7 @@ __global__ __launch_bounds__(256) void k_plain_narrow(Planes B, const float *ver
     for (int base = blockIdx.x * range; base < total; base += gridDim.x * range) {
         const int count = min(range, total - base);
         WorldSrc<false> src{B, verts, nb, ns, &fl, cand + base, rec + base, flag + base, cnt, PairDecode32{}};
-        narrow_block<256, false>(src, count, np, lds, sh, qidx + base, qsim + base);
+        narrow_block<256>(src, count, np, lds, sh, qidx + base, qsim + base);
         if (threadIdx.x == 0) {
             atomicAdd(&cnt[CNT_GJK_FOUND], (unsigned long long)sh.nepa);
             if (sh.stalled) atomicAdd(&cnt[CNT_EPA_OVERFLOW], (unsigned long long)sh.stalled);
@@ -802,7 +802,7 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
     // narrowphase over the candidates (GJK per lane, EPA per wave)
     {
         WorldSrc<true> src{Lb, vertsL, nb, ns, &fl, cand, rec, flag, a.cnt, dec};
-        narrow_team<false, ISL>(t, src, ncand, a.k.np, epa, nsh, S.qidx, S.qsim);
+        narrow_team<ISL>(t, src, ncand, a.k.np, epa, nsh, S.qidx, S.qsim);
     }
     if (tid == 0) {
         atomicAdd(&a.cnt[CNT_GJK_FOUND], (unsigned long long)nsh.nepa);
