@@ -314,7 +314,7 @@ __device__ inline double face_dist64(const EpaLds &L, const FaceR &f)
 // caller has written the GJK simplex to L.vp / L.va / L.vb[0..3], passes vertex
 // (lane)'s P in p0 for lanes 0-3, and has called wave_sync().  Every lane returns
 // the same result.
-__device__ inline EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, const NarrowParams &p)
+__device__ __forceinline__ EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, const NarrowParams &p)
 {
     const int lane = lane_id();
     EpaResult r;
@@ -870,7 +870,7 @@ __device__ inline void group_argmin64(bool &valid, double &v, int &i)
 // ISL: the FP64-islands mode, whose final face choice and depth are binary64
 // (as epa_wave's).
 template <int G, bool ISL = false>
-__device__ inline EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0, V3 sb0, bool act,
+__device__ __forceinline__ EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0, V3 sb0, bool act,
                                       const NarrowParams &p)
 {
     const int lane = lane_id(), j = lane & (G - 1), gb = lane & (64 - G), g = lane / G;
@@ -1217,7 +1217,7 @@ struct GjkLane {
 
 // Candidate c for the lane (c >= ncand: none left, the lane retires).
 template <class Src>
-__device__ inline void gjk_lane_take(GjkLane &G, const Src &src, int c, int ncand, float *cyc)
+__device__ __forceinline__ void gjk_lane_take(GjkLane &G, const Src &src, int c, int ncand, float *cyc)
 {
     if (c >= ncand) {
         G.retired = true;
@@ -1239,7 +1239,7 @@ __device__ inline void gjk_lane_take(GjkLane &G, const Src &src, int c, int ncan
 // One EvolveSimplex call of the lane's candidate, with the cycle check: the
 // outcome once the loop has ended (GJK_NO, GJK_FOUND, or GJK_CAP at the 65-call
 // cap), else GJK_STILL.
-__device__ inline int gjk_lane_call(GjkLane &G, float *cyc, const NarrowParams &np)
+__device__ __forceinline__ int gjk_lane_call(GjkLane &G, float *cyc, const NarrowParams &np)
 {
     const int tid = lane_id();
     Simplex &S = G.S;
@@ -1282,7 +1282,7 @@ __device__ inline int gjk_lane_call(GjkLane &G, float *cyc, const NarrowParams &
 // in binary64); without it, that mode runs every polytope by the whole wave.
 // The team's wave k uses epa[k]; sh, qidx and qsim are the team's own.
 template <bool ISL = false, class Src>
-__device__ void narrow_team(const Team &team, const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
+__device__ __forceinline__ void narrow_team(const Team &team, const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
                             NarrowShared &sh, int *qidx, SimplexRec *qsim)
 {
     const bool grouped = ISL || !np.fp64_islands;
