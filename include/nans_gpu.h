@@ -205,12 +205,9 @@ int nans_download_state(nans_ctx *ctx, nans_bodies_soa *bodies);
  * statistics), with the warm-start lists emptied. */
 int nans_step_plain(nans_ctx *ctx, int32_t nsteps);
 
-/* Advance every world by nsteps with the batched path: one persistent launch per
- * step over all worlds (at most 512 bodies per world).  The step (work-counter
- * reset + step kernel) is captured once in a hipGraph and replayed nsteps times;
- * the graph is kept until the batch, the parameters or the tuning change.  With
- * the warm start on (nans_set_warm_start), the warm-started step kernel is
- * launched step by step instead. */
+/* Advance every world by nsteps with the batched path (at most 512 bodies per
+ * world): one persistent launch per call (per 256 steps of a longer one), in which
+ * a world's steps run one after another on the workgroup that took it. */
 int nans_step_batched(nans_ctx *ctx, int32_t nsteps);
 
 /* Device time of the last nans_step_batched call, from HIP events recorded on
@@ -227,9 +224,8 @@ typedef struct nans_timing {
 int nans_batched_timing(nans_ctx *ctx, nans_timing *timing);
 
 /* Overwrite pos, vel, angvel, angles (and force, torque; NULL = zero) of the
- * uploaded batch in place, keeping buffers and the captured graph.  The
- * quaternions of the opt-in orientation mode are set from the given angles, as
- * nans_upload_worlds sets them. */
+ * uploaded batch in place, keeping its buffers.  The quaternions of the opt-in
+ * orientation mode are set from the given angles, as nans_upload_worlds sets them. */
 int nans_set_state(nans_ctx *ctx, const nans_bodies_soa *bodies);
 
 /* Orientation of both steps.  EULER (the default) is the reference's: Angles in
@@ -261,8 +257,7 @@ int nans_get_quaternions(nans_ctx *ctx, float *quat);
  * unchanged.  At most 16 n + 64 contacts of a world carry over; the others start
  * from zero.  Enabling it, nans_set_state and nans_upload_worlds empty the
  * lists.  Results differ from the reference's by design.  The plain and the
- * batched step share the lists, so the two can alternate; the batched step then
- * launches step by step instead of replaying its graph.  The autotuner and the
+ * batched step share the lists, so the two can alternate.  The autotuner and the
  * differentiable rollout refuse the mode. */
 int nans_set_warm_start(nans_ctx *ctx, int32_t enable);
 

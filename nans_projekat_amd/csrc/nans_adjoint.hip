@@ -27,11 +27,10 @@
 namespace nans {
 
 enum : int { ADJ_CNT_OVERFLOW = 0, ADJ_CNT_REPLAY, ADJ_CNT_N };
-constexpr int ST_FIELDS = 18;  // kept state: P V W A (12 planes) then F T (6 planes)
 
 struct AdjArgs {
-    const float *state;   // [ST_FIELDS][N] at the start of the step
-    const float *next;    // [ST_FIELDS][N] after it
+    const float *state;   // [STATE_FIELDS][N] at the start of the step
+    const float *next;    // [STATE_FIELDS][N] after it
     const float *planes;  // the batch's planes (scale, mass, moi)
     int64_t N;
     const int *offsets;
@@ -248,11 +247,11 @@ __global__ void k_adj_zero_u64(unsigned long long *p, int n)
 struct AdjointTape {
     int steps = 0, every = 0, ncp = 0;
     nans_params params;
-    float *cp = nullptr;        // [ncp][ST_FIELDS][N]
-    float *last = nullptr;      // [ST_FIELDS][N] after the rollout
+    float *cp = nullptr;        // [ncp][STATE_FIELDS][N]
+    float *last = nullptr;      // [STATE_FIELDS][N] after the rollout
     // backward scratch
     int seg_len = 0;
-    float *seg = nullptr;       // [seg_len + 1][ST_FIELDS][N]
+    float *seg = nullptr;       // [seg_len + 1][STATE_FIELDS][N]
     ContactRec *seg_rec = nullptr;  // [seg_len][total]
     int *seg_cnt = nullptr;     // [seg_len][nworlds]
     AdjTape *tape = nullptr;    // [total]
@@ -286,7 +285,7 @@ void adjoint_release(nans_worlds *W)
     W->adj = nullptr;
 }
 
-// state planes <-> a kept slot [ST_FIELDS][N]
+// state planes <-> a kept slot [STATE_FIELDS][N]
 static int save_state(nans_worlds *W, float *dst, hipStream_t s)
 {
     const size_t N = (size_t)W->N;
@@ -343,7 +342,7 @@ int nans_rollout(nans_ctx *ctx, int32_t nsteps, int32_t checkpoint_every)
     NANS_HIP(hipStreamSynchronize(s));
     if (!W->adj) W->adj = new AdjointTape();
     AdjointTape *T = W->adj;
-    const size_t slot = (size_t)ST_FIELDS * W->N;
+    const size_t slot = (size_t)STATE_FIELDS * W->N;
     const int ncp = (nsteps + checkpoint_every - 1) / checkpoint_every;
     if (ncp != T->ncp || !T->cp) {
         wfree(T->cp);
@@ -384,7 +383,7 @@ int nans_adjoint(nans_ctx *ctx, const nans_adjoint_io *io)
     NANS_HIP(hipStreamSynchronize(s));
     const int64_t N = W->N;
     const int nw = W->nworlds;
-    const size_t slot = (size_t)ST_FIELDS * N;
+    const size_t slot = (size_t)STATE_FIELDS * N;
     // contact capacity per world and step, as the contact recording of the step
     if (!T->rec_off) {
         std::vector<int64_t> off(nw + 1, 0);
@@ -457,13 +456,10 @@ int nans_adjoint(nans_ctx *ctx, const nans_adjoint_io *io)
         const int t0 = j * T->every;
         const int len = std::min(T->every, T->steps - t0);
         rc = load_state(W, T->cp + slot * j, s);
-        for (int st = 0; st < len && rc == NANS_OK; ++st) {
-            rc = save_state(W, T->seg + slot * st, s);
-            if (rc == NANS_OK)
-                rc = batched_step_recorded(ctx, s, T->seg_rec + (size_t)T->total * st, T->rec_off,
-                                           T->seg_cnt + (size_t)nw * st, T->rec_cap);
-        }
-        if (rc == NANS_OK) rc = save_state(W, T->seg + slot * len, s);
+        if (rc == NANS_OK) rc = save_state(W, T->seg, s);
+        if (rc == NANS_OK)
+            rc = batched_run_recorded(ctx, len, s,
+                                      BatchRecord{T->seg, T->seg_rec, T->total, T->rec_off, T->seg_cnt, T->rec_cap});
         for (int st = len - 1; st >= 0 && rc == NANS_OK; --st) {
             a.state = T->seg + slot * st;
             a.next = T->seg + slot * (st + 1);

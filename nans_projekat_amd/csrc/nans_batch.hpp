@@ -33,7 +33,10 @@ enum : int {
     CNT_N
 };
 
-// Arguments of k_batched_step (one persistent launch = one step of every world).
+// A kept state: planes P V W A (the first F_SX fields), then force and torque.
+constexpr int STATE_FIELDS = F_SX + 6;
+
+// Arguments of k_batched_step (one persistent launch = nsteps steps of every world).
 struct BatchArgs {
     float *planes;          // [F_NFIELDS][N]
     int64_t N;
@@ -45,8 +48,9 @@ struct BatchArgs {
     int nmax;               // LDS stride of a workgroup's world (>= largest world)
     int wrows;              // LDS stride of a wave's world (>= largest of order[nbig, nworlds))
     int lds_floats;         // floats of world LDS before the polytope LDS (a multiple of 4)
-    int *queue;             // this step's work counters: [0] workgroup worlds, [1] wave worlds
-    int *queue_next;        // the next step's counters, cleared by this launch (or null)
+    int nsteps;
+    int *queue;             // this launch's work counters: [0] workgroup worlds, [1] wave worlds
+    int *queue_next;        // the next launch's counters, cleared by this one
     StepConsts k;
     const FloorDev *fl;
     const float *wfric, *wrest;  // per-world coefficients (may be null)
@@ -59,9 +63,12 @@ struct BatchArgs {
     int wcap;               // entries per wave in the wave phase (cap / waves)
     float *corners;         // per-workgroup box corners, corner_stride floats each
     int64_t corner_stride;
-    ContactRec *rec_out;    // recording (may be null)
-    const int64_t *rec_off;
+    float *state_out;       // [nsteps + 1][STATE_FIELDS][N]: slot k + 1 receives the state after step k (may be null)
+    ContactRec *rec_out;    // recording (may be null): step k's contacts of world w at
+    int64_t rec_stride;     // k * rec_stride + rec_off[w], their number at
+    const int64_t *rec_off; // rec_count[k * rec_count_stride + w]
     int *rec_count;
+    int rec_count_stride;
     const int *rec_cap;
     unsigned long long *cnt;
 };
@@ -74,12 +81,10 @@ template <bool WARM>
 struct BatchArgsT : BatchArgs {};
 template <>
 struct BatchArgsT<true> : BatchArgs {
-    const int *warm_p_prev = nullptr;
-    const float *warm_s_prev = nullptr;
-    const int *warm_n_prev = nullptr;
-    int *warm_p_next = nullptr;
-    float *warm_s_next = nullptr;
-    int *warm_n_next = nullptr;
+    int *warm_p0 = nullptr, *warm_p1 = nullptr;  // step k reads the lists of buffer (warm_flip + k) & 1
+    float *warm_s0 = nullptr, *warm_s1 = nullptr;  // and writes the other's
+    int *warm_n0 = nullptr, *warm_n1 = nullptr;
+    int warm_flip = 0;
     const int64_t *warm_off = nullptr;
     const int *warm_cap = nullptr;
 };
@@ -106,16 +111,21 @@ int check_overflow(nans_ctx *ctx);
 // (and empties the warm-start lists) before returning NANS_ERR_CAPACITY.
 int snapshot_take(nans_ctx *ctx, hipStream_t s);
 int step_finish(nans_ctx *ctx);
-// nsteps batched steps replayed from the captured one-step graph
+// nsteps batched steps (warm-started if the context is)
 int batched_run(nans_ctx *ctx, int nsteps, int block);
 // threads per world of the batched step (the autotuner's choice or the default)
 int batched_block(nans_ctx *ctx);
-// One batched step launched directly on stream s, recording every world's
-// contact list into rec_out (per-world offsets rec_off, capacities rec_cap,
-// counts rec_count).
-int batched_step_recorded(nans_ctx *ctx, hipStream_t s, ContactRec *rec_out, const int64_t *rec_off,
-                          int *rec_count, const int *rec_cap);
-
+// Where a run of cold batched steps keeps every step's state and contact lists
+// (BatchArgs' recording fields).
+struct BatchRecord {
+    float *state;
+    ContactRec *rec;
+    int64_t rec_stride;
+    const int64_t *rec_off;
+    int *rec_count;  // nworlds per step
+    const int *rec_cap;
+};
+int batched_run_recorded(nans_ctx *ctx, int nsteps, hipStream_t s, const BatchRecord &rec);
 
 }  // namespace nans
 
@@ -206,6 +216,7 @@ struct nans_worlds {
     int64_t b_corner_floats = 0;   // its size
     int *queue = nullptr;
     int queue_len = 0;
+    int queue_flip = 0;  // which half of queue[] the next batched launch uses
     // recording
     int record = 0;
     nans::ContactRec *rec_buf = nullptr;
@@ -214,17 +225,11 @@ struct nans_worlds {
     int *rec_cap = nullptr;
     std::vector<int64_t> h_rec_off;
     std::vector<int> h_rec_cap;
-    // graph cache of the batched step
-    hipGraphExec_t graph = nullptr;   // two steps, on counter buffers A then B
-    hipGraphExec_t graph1 = nullptr;  // one step, on buffer A
-    int graph_steps = -1;
-    int graph_block = 0;
-    nans_params graph_params;
-    int graph_orientation = 0;
-    hipEvent_t ev_in = nullptr, ev_out = nullptr, ev_t0 = nullptr, ev_t1 = nullptr;
-    int graph_grid = 0, graph_lds = 0;
-    int graph_wave = -1;     // worlds of at most this many bodies ran one per wave
-    int graph_nwave = 0;     // and there were this many of them
+    hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr;
+    // shape of the last batched launch
+    int shape_block = 0, shape_grid = 0, shape_lds = 0;
+    int shape_wave = -1;     // worlds of at most this many bodies ran one per wave
+    int shape_nwave = 0;     // and there were this many of them
     int timed_steps = 0;
     float timed_ms = 0.0f;
     int tuned_block = 0;   // autotuner's choice of threads per world (0: not tuned)

@@ -236,15 +236,8 @@ int nans_create(nans_ctx **out, const nans_params *p)
         delete c;
         return rc;
     }
-    hipError_t e = hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking);
+    hipError_t e = hipMalloc((void **)&c->d_counters, 64 * sizeof(unsigned long long));
     if (e != hipSuccess) {
-        delete c;
-        set_error("hipStreamCreateWithFlags: %s", hipGetErrorString(e));
-        return NANS_ERR_HIP;
-    }
-    e = hipMalloc((void **)&c->d_counters, 64 * sizeof(unsigned long long));
-    if (e != hipSuccess) {
-        hipStreamDestroy(c->own_stream);
         delete c;
         set_error("hipMalloc: %s", hipGetErrorString(e));
         return NANS_ERR_HIP;
@@ -262,7 +255,6 @@ int nans_destroy(nans_ctx *ctx)
     hipFree(ctx->d_counters);
     if (ctx->np_qidx) hipFree(ctx->np_qidx);
     if (ctx->np_qsim) hipFree(ctx->np_qsim);
-    hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return NANS_OK;
 }

@@ -61,7 +61,6 @@ int worlds_release(nans_ctx *ctx);  // frees the world batch of a context
 struct nans_ctx {
     nans_params p;
     hipStream_t stream;          // stream the calls are ordered on
-    hipStream_t own_stream;      // private stream for graph capture / replay
     unsigned long long *d_counters;  // small device scratch counters
     nans_worlds *worlds;
     int64_t np_cap;                  // narrowphase entry point: queue capacity (pairs)

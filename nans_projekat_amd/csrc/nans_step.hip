@@ -10,9 +10,9 @@
 // Two launch structures share the device routines of nans_world.hpp:
 //   plain    one world per launch sequence, grid-wide kernels:
 //            forces+corners | cull count | scan | cull write | narrowphase | solve
-//   batched  one persistent launch per step; each workgroup takes worlds from a
-//            queue (largest first) and runs the whole step of a world with its
-//            bodies in LDS; the steps of a call are captured in a hipGraph.
+//   batched  one persistent launch per call; each workgroup takes worlds from a
+//            queue (largest first) and runs every step of a world with its bodies
+//            in LDS.
 //
 // SolveConstraints applies the contacts one after another in list order
 // (code/nans.cpp:1541-1547), each reading the velocities left by the previous
@@ -634,10 +634,10 @@ struct WorldScratch {
     int cap;
 };
 
-// The whole step of world w by team t (the workgroup, or one wave of it): epa[k]
-// is the polytope LDS of the team's wave k, wave_tot one int per wave.
+// Step number step of the launch for world w by team t (the workgroup, or one wave
+// of it): epa[k] is the polytope LDS of the team's wave k, wave_tot one int per wave.
 template <int BLOCK, bool WARM, bool ISL>
-__device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const Team &t, int w, const WorldLds &L,
+__device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const Team &t, int w, int step, const WorldLds &L,
                                               const WorldScratch &S, EpaLds *epa, NarrowShared &nsh,
                                               int *wave_tot, const FloorDev &fl)
 {
@@ -832,9 +832,10 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
     float *wsum = reinterpret_cast<float *>(rec);  // [3 ncon]
     if constexpr (WARM) {
         const int64_t off = a.warm_off[w];
-        const int *pp = a.warm_p_prev + off;
-        const float *sp = a.warm_s_prev + 3 * off;
-        const int np = a.warm_n_prev[w];
+        const bool odd = (a.warm_flip + step) & 1;
+        const int *pp = (odd ? a.warm_p1 : a.warm_p0) + off;
+        const float *sp = (odd ? a.warm_s1 : a.warm_s0) + 3 * off;
+        const int np = (odd ? a.warm_n1 : a.warm_n0)[w];
         for (int c = tid; c < ncon; c += T) {
             const int key = cand[c];
             int lo = 0, hi = np;
@@ -860,12 +861,15 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
                                       WARM ? wsum : nullptr);
     if constexpr (WARM) {  // this step's list: the first warm_cap[w] contacts (contact c's sums are team thread c % T's)
         const int64_t off = a.warm_off[w];
+        const bool odd = (a.warm_flip + step) & 1;
+        int *pn = (odd ? a.warm_p0 : a.warm_p1) + off;
+        float *sn = (odd ? a.warm_s0 : a.warm_s1) + 3 * off;
         const int m = min(ncon, a.warm_cap[w]);
         for (int c = tid; c < m; c += T) {
-            a.warm_p_next[off + c] = cand[c];
-            for (int q = 0; q < 3; ++q) a.warm_s_next[3 * (off + c) + q] = wsum[3 * c + q];
+            pn[c] = cand[c];
+            for (int q = 0; q < 3; ++q) sn[3 * c + q] = wsum[3 * c + q];
         }
-        if (tid == 0) a.warm_n_next[w] = m;
+        if (tid == 0) (odd ? a.warm_n0 : a.warm_n1)[w] = m;
     }
     // IntegrateVelocities and write-back
     for (int i = tid; i < n; i += T) {
@@ -873,19 +877,30 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
         else integrate_velocities_body(Lb, i, a.k.dt);
 #pragma unroll
         for (int f = 0; f < F_SX; ++f) Gw.at(f, i) = Lb.at(f, i);
+        if (a.state_out) {  // the state after the step: F_SX planes, then force and torque, now zero
+            const Planes K{a.state_out + (int64_t)(step + 1) * STATE_FIELDS * a.N + b0, (int)a.N};
+#pragma unroll
+            for (int f = 0; f < F_SX; ++f) K.at(f, i) = Lb.at(f, i);
+#pragma unroll
+            for (int f = F_SX; f < STATE_FIELDS; ++f) K.at(f, i) = 0.0f;
+        }
     }
     if (a.rec_out) {
-        ContactRec *dst = a.rec_out + a.rec_off[w];
+        ContactRec *dst = a.rec_out + step * a.rec_stride + a.rec_off[w];
         int rc = a.rec_cap[w];
         for (int c = tid; c < ncon && c < rc; c += T) dst[c] = con[c];
-        if (tid == 0) a.rec_count[w] = ncon;
+        if (tid == 0) a.rec_count[(int64_t)step * a.rec_count_stride + w] = ncon;
     }
     t.sync();
 }
 
-// The persistent step: the worlds order[0, nbig) (the larger ones, largest
-// first) each by a whole workgroup, then order[nbig, nworlds) each by one wave,
-// every wave of a workgroup taking its own.  Each phase hands out its worlds
+// Persistent launch of nsteps steps: the worlds order[0, nbig) (the larger ones,
+// largest first) each by a whole workgroup, then order[nbig, nworlds) each by one
+// wave, every wave of a workgroup taking its own.  Worlds do not touch each other,
+// so a team runs every step of its world before it takes another: a launch per
+// step ended with the slowest world of that step (1024 worlds of 16 bodies, rollout
+// and gradient of 240 steps: 94.1 -> 68.3 ms; 4096 worlds of 8-256, 60 steps: 85.4
+// -> 81.0 ms; 601 with warm start, 30 steps: 38.8 -> 34.2 ms).  Each phase hands out its worlds
 // from its own counter (queue[0], queue[1]).
 // WARM: the opt-in warm start, each contact's accumulators carried over from the
 // world's previous step (a separate instantiation; the default step has none of it).
@@ -909,8 +924,8 @@ k_batched_step(BatchArgsT<WARM> a)
     const FloorDev &fl = *a.fl;  // in global memory, as the box corners
     __shared__ NarrowShared nsh[NW];
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    // the next launch's counters: no launch of this step reads them
-    if (a.queue_next && blockIdx.x == 0 && threadIdx.x == 0) {
+    // the next launch's counters: this one does not read them
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
         a.queue_next[0] = 0;
         a.queue_next[1] = 0;
     }
@@ -924,31 +939,37 @@ k_batched_step(BatchArgsT<WARM> a)
     EpaLds *tepa = epa;
     int tsh = 0;
     bool whole = true;
+    // one loop over the steps of all jobs (a step loop inside the job loop had the
+    // compiler hoist the world's terms and spill 91 registers for it)
+    int job = 0, step = a.nsteps;
     for (;;) {
-        int job = 0;
-        if (whole) {
-            if (threadIdx.x == 0) s_job = atomicAdd(&a.queue[0], 1);
-            __syncthreads();
-            job = __builtin_amdgcn_readfirstlane(s_job);
-            __syncthreads();
-            if (job >= a.nbig) {  // the wave phase: each wave its own LDS part and scratch
-                whole = false;
-                t = Team::wave();
-                L = world_lds(smem + wv * world_lds_floats(a.wrows), a.wrows,
-                              corners + wv * world_corner_floats(a.wrows));
-                const int64_t o = wg + (int64_t)wv * a.wcap;
-                S = WorldScratch{a.cand + o, a.rec + o, a.flag + o, a.qidx + o, a.qsim + o, a.wcap};
-                tepa = epa + wv;
-                tsh = wv;
+        if (step == a.nsteps) {
+            step = 0;
+            if (whole) {
+                if (threadIdx.x == 0) s_job = atomicAdd(&a.queue[0], 1);
+                __syncthreads();
+                job = __builtin_amdgcn_readfirstlane(s_job);
+                __syncthreads();
+                if (job >= a.nbig) {  // the wave phase: each wave its own LDS part and scratch
+                    whole = false;
+                    t = Team::wave();
+                    L = world_lds(smem + wv * world_lds_floats(a.wrows), a.wrows,
+                                  corners + wv * world_corner_floats(a.wrows));
+                    const int64_t o = wg + (int64_t)wv * a.wcap;
+                    S = WorldScratch{a.cand + o, a.rec + o, a.flag + o, a.qidx + o, a.qsim + o, a.wcap};
+                    tepa = epa + wv;
+                    tsh = wv;
+                }
             }
+            if (!whole) {
+                int j = 0;
+                if ((threadIdx.x & 63) == 0) j = atomicAdd(&a.queue[1], 1);
+                job = a.nbig + __builtin_amdgcn_readfirstlane(j);
+            }
+            if (job >= a.nworlds) break;
         }
-        if (!whole) {
-            int j = 0;
-            if ((threadIdx.x & 63) == 0) j = atomicAdd(&a.queue[1], 1);
-            job = a.nbig + __builtin_amdgcn_readfirstlane(j);
-        }
-        if (job >= a.nworlds) break;
-        batched_world<BLOCK, WARM, ISL>(a, t, a.order[job], L, S, tepa, nsh[tsh], wave_tot, fl);
+        batched_world<BLOCK, WARM, ISL>(a, t, a.order[job], step, L, S, tepa, nsh[tsh], wave_tot, fl);
+        ++step;
     }
 }
 
@@ -975,20 +996,9 @@ void wfree(void *p)
     if (p) (void)hipFree(p);
 }
 
-static void drop_graph(nans_worlds *W)
-{
-    if (W->graph) (void)hipGraphExecDestroy(W->graph);
-    if (W->graph1) (void)hipGraphExecDestroy(W->graph1);
-    W->graph = nullptr;
-    W->graph1 = nullptr;
-    W->graph_steps = -1;
-}
-
-// Frees the batched step's per-workgroup scratch, and with it the captured graph,
-// whose kernel arguments point into that scratch.
+// Frees the batched step's per-workgroup scratch.
 static void release_batch_scratch(nans_worlds *W)
 {
-    drop_graph(W);
     wfree(W->b_cand);
     wfree(W->b_rec);
     wfree(W->b_flag);
@@ -1036,7 +1046,6 @@ int worlds_release(nans_ctx *ctx)
 {
     if (!ctx || !ctx->worlds) return NANS_OK;
     nans_worlds *W = ctx->worlds;
-    drop_graph(W);
     for (void *p : {(void *)W->planes, (void *)W->verts, (void *)W->brad, (void *)W->offsets, (void *)W->nboxes,
                     (void *)W->order, (void *)W->wfric, (void *)W->wrest, (void *)W->floor, (void *)W->cnt,
                     (void *)W->cand, (void *)W->rec, (void *)W->flag, (void *)W->con, (void *)W->done,
@@ -1048,7 +1057,7 @@ int worlds_release(nans_ctx *ctx)
                     (void *)W->warm_s[1], (void *)W->warm_n[0], (void *)W->warm_n[1], (void *)W->warm_cp,
                     (void *)W->warm_sums, (void *)W->warm_offd, (void *)W->warm_capd, (void *)W->snap})
         wfree(p);
-    for (hipEvent_t ev : {W->ev_in, W->ev_out, W->ev_t0, W->ev_t1})
+    for (hipEvent_t ev : {W->ev_t0, W->ev_t1})
         if (ev) (void)hipEventDestroy(ev);
     release_batch_scratch(W);
     release_recording(W);
@@ -1496,7 +1505,6 @@ int nans_record_contacts(nans_ctx *ctx, int32_t enable)
     NANS_HIP(hipDeviceSynchronize());
     nans_worlds *W = ctx->worlds;
     W->record = enable ? 1 : 0;
-    drop_graph(W);
     if (W->record) return alloc_recording(ctx);
     release_recording(W);
     return NANS_OK;
@@ -1746,8 +1754,7 @@ static int batched_config(nans_ctx *ctx, const WaveSplit &sp, int *grid, size_t 
 
 // Launch shape, per-workgroup scratch and kernel arguments of the batched step.
 template <int BLOCK, bool WARM, bool ISL>
-static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *lds_out,
-                           WaveSplit *split_out = nullptr)
+static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *lds_out)
 {
     nans_worlds *W = ctx->worlds;
     int grid = 0;
@@ -1769,15 +1776,15 @@ static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *l
         W->b_grid = grid;
         W->b_cap = (int)cap;
     }
-    // two buffers of work counters, A = queue[0, 2) and B = queue[2, 4), zero here;
-    // every call leaves A zero (B is cleared by the launch before the one using it)
+    // two buffers of work counters, queue[0, 2) and queue[2, 4): a launch takes its
+    // jobs from the one at 2 * queue_flip, zero by then, and clears the other
     if (W->queue_len < 4) {
-        drop_graph(W);
         wfree(W->queue);
         W->queue = nullptr;
         NANS_TRY(dmalloc(&W->queue, 4));
         NANS_HIP(hipMemset(W->queue, 0, sizeof(int) * 4));
         W->queue_len = 4;
+        W->queue_flip = 0;
     }
     a.planes = W->planes;
     a.N = W->N;
@@ -1803,7 +1810,6 @@ static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *l
     // box corners: a workgroup world's, or its waves' worlds side by side
     a.corner_stride = std::max(world_corner_floats(W->nmax), NW * world_corner_floats(sp.wrows));
     if (W->b_corner_floats < a.corner_stride * grid) {
-        drop_graph(W);
         wfree(W->b_corners);
         W->b_corners = nullptr;
         W->b_corner_floats = 0;
@@ -1811,59 +1817,67 @@ static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *l
         W->b_corner_floats = a.corner_stride * grid;
     }
     a.corners = W->b_corners;
-    a.rec_out = W->record ? W->rec_buf : nullptr;
+    a.state_out = nullptr;
+    a.rec_out = W->record ? W->rec_buf : nullptr;  // the last step's contacts stay
+    a.rec_stride = 0;
     a.rec_off = W->rec_off;
     a.rec_count = W->rec_count;
+    a.rec_count_stride = 0;
     a.rec_cap = W->rec_cap;
     a.cnt = W->cnt;
-    a.queue = W->queue;
-    a.queue_next = nullptr;
-    if (split_out) *split_out = sp;
+    W->shape_block = BLOCK;
+    W->shape_grid = grid;
+    W->shape_lds = (int)lds;
+    W->shape_wave = sp.bodies;
+    W->shape_nwave = sp.nwave;
     *grid_out = grid;
     *lds_out = lds;
     return NANS_OK;
 }
 
-template <int BLOCK, bool ISL>
-static int batched_capture(nans_ctx *ctx, int nsteps, hipStream_t cs)
+// Steps of one launch of the batched kernel: a launch keeps a bounded length, and
+// beyond a few dozen steps the worlds' times even out anyway.
+constexpr int BATCH_LAUNCH_STEPS = 256;
+
+// nsteps steps on stream s; rec: where to keep every step's state and contacts, or
+// null (one launch: nsteps is then at most BATCH_LAUNCH_STEPS).
+template <int BLOCK, bool WARM, bool ISL>
+static int batched_launches(nans_ctx *ctx, int nsteps, hipStream_t s, const BatchRecord *rec)
 {
     nans_worlds *W = ctx->worlds;
-    BatchArgsT<false> a;
+    BatchArgsT<WARM> a;
     int grid = 0;
     size_t lds = 0;
-    WaveSplit sp;
-    NANS_TRY((batched_prepare<BLOCK, false, ISL>(ctx, a, &grid, &lds, &sp)));
-    // two steps: the step kernel on counter buffer A, clearing B, then on B, clearing
-    // A (no clearing kernel or memset node per step); and one step on A, after which
-    // the caller clears A.  A call of nsteps replays the first graph nsteps / 2 times
-    // and the second once if nsteps is odd.
-    int *const qa = W->queue, *const qb = W->queue + 2;
-    auto capture = [&](hipGraphExec_t *out, int steps) -> int {
-        hipGraph_t g = nullptr;
-        NANS_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < steps; ++k) {
-            a.queue = k ? qb : qa;
-            a.queue_next = steps == 1 ? nullptr : (k ? qa : qb);
-            k_batched_step<BLOCK, false, ISL><<<grid, BLOCK, lds, cs>>>(a);
-        }
-        hipError_t e = hipStreamEndCapture(cs, &g);
-        NANS_REQUIRE(e == hipSuccess, NANS_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
-        e = hipGraphInstantiate(out, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        NANS_REQUIRE(e == hipSuccess, NANS_ERR_HIP, "graph instantiate failed: %s", hipGetErrorString(e));
-        return NANS_OK;
-    };
-    drop_graph(W);
-    NANS_TRY(capture(&W->graph, 2));
-    NANS_TRY(capture(&W->graph1, 1));
-    W->graph_steps = nsteps;
-    W->graph_block = BLOCK;
-    W->graph_params = ctx->p;
-    W->graph_orientation = ctx->orientation;
-    W->graph_grid = grid;
-    W->graph_lds = (int)lds;
-    W->graph_wave = sp.bodies;
-    W->graph_nwave = sp.nwave;
+    NANS_TRY((batched_prepare<BLOCK, WARM, ISL>(ctx, a, &grid, &lds)));
+    if (rec) {
+        a.state_out = rec->state;
+        a.rec_out = rec->rec;
+        a.rec_stride = rec->rec_stride;
+        a.rec_off = rec->rec_off;
+        a.rec_count = rec->rec_count;
+        a.rec_count_stride = W->nworlds;
+        a.rec_cap = rec->rec_cap;
+    }
+    if constexpr (WARM) {
+        a.warm_p0 = W->warm_p[0];
+        a.warm_p1 = W->warm_p[1];
+        a.warm_s0 = W->warm_s[0];
+        a.warm_s1 = W->warm_s[1];
+        a.warm_n0 = W->warm_n[0];
+        a.warm_n1 = W->warm_n[1];
+        a.warm_off = W->warm_offd;
+        a.warm_cap = W->warm_capd;
+    }
+    for (int done = 0; done < nsteps; done += a.nsteps) {
+        a.nsteps = std::min(nsteps - done, BATCH_LAUNCH_STEPS);
+        a.queue = W->queue + 2 * W->queue_flip;
+        a.queue_next = W->queue + 2 * (W->queue_flip ^ 1);
+        if constexpr (WARM) a.warm_flip = W->warm_flip;
+        k_batched_step<BLOCK, WARM, ISL><<<grid, BLOCK, lds, s>>>(a);
+        NANS_HIP(hipGetLastError());
+        W->queue_flip ^= 1;
+        if constexpr (WARM) W->warm_flip = (W->warm_flip + a.nsteps) & 1;
+    }
     return NANS_OK;
 }
 
@@ -1873,99 +1887,21 @@ int batched_run(nans_ctx *ctx, int nsteps, int block)
     NANS_REQUIRE(W->nmax <= BATCH_MAX_BODIES, NANS_ERR_CAPACITY,
                  "the batched step keeps a world in LDS: at most %d bodies per world (largest: %d)",
                  BATCH_MAX_BODIES, W->nmax);
-    hipStream_t cs = ctx->own_stream;
-    if (!W->ev_in) {
-        NANS_HIP(hipEventCreateWithFlags(&W->ev_in, hipEventDisableTiming));
-        NANS_HIP(hipEventCreateWithFlags(&W->ev_out, hipEventDisableTiming));
+    hipStream_t s = ctx->stream;
+    if (!W->ev_t0) {
         NANS_HIP(hipEventCreate(&W->ev_t0));
         NANS_HIP(hipEventCreate(&W->ev_t1));
     }
-    bool reuse = W->graph && W->graph_block == block && W->graph_wave == wave_bodies(W, block) &&
-                 W->graph_orientation == ctx->orientation &&
-                 memcmp(&W->graph_params, &ctx->p, sizeof(nans_params)) == 0;
-    if (!reuse) {
-        NANS_TRY(setup_floor(ctx, ctx->stream));
-        NANS_HIP(hipStreamSynchronize(ctx->stream));
-        NANS_TRY(by_shape(block, ctx->p.fp64_islands != 0, [&](auto B, auto I) {
-            return batched_capture<decltype(B)::value, decltype(I)::value>(ctx, 1, cs);
-        }));
-    }
-    NANS_HIP(hipEventRecord(W->ev_in, ctx->stream));
-    NANS_HIP(hipStreamWaitEvent(cs, W->ev_in, 0));
-    // events on the stream the kernels run on bracket the nsteps graph launches
-    NANS_HIP(hipEventRecord(W->ev_t0, cs));
-    int s = 0;
-    for (; s + 2 <= nsteps; s += 2) NANS_HIP(hipGraphLaunch(W->graph, cs));
-    if (s < nsteps) {
-        NANS_HIP(hipGraphLaunch(W->graph1, cs));
-        k_zero_i32<<<1, 64, 0, cs>>>(W->queue, 2);  // A zero again for the next call
-    }
-    NANS_HIP(hipEventRecord(W->ev_t1, cs));
-    NANS_HIP(hipEventRecord(W->ev_out, cs));
-    NANS_HIP(hipStreamWaitEvent(ctx->stream, W->ev_out, 0));
-    W->timed_steps = nsteps;
-    return NANS_OK;
-}
-
-// The warm-started batched step: launched step by step (no graph), since each
-// step swaps the previous and next contact lists.
-template <int BLOCK, bool ISL>
-static int batched_warm_launches(nans_ctx *ctx, int nsteps, hipStream_t cs)
-{
-    nans_worlds *W = ctx->worlds;
-    BatchArgsT<true> a;
-    int grid = 0;
-    size_t lds = 0;
-    WaveSplit sp;
-    NANS_TRY((batched_prepare<BLOCK, true, ISL>(ctx, a, &grid, &lds, &sp)));
-    a.warm_off = W->warm_offd;
-    a.warm_cap = W->warm_capd;
-    for (int s = 0; s < nsteps; ++s) {
-        const int cur = W->warm_flip, nxt = cur ^ 1;
-        a.warm_p_prev = W->warm_p[cur];
-        a.warm_s_prev = W->warm_s[cur];
-        a.warm_n_prev = W->warm_n[cur];
-        a.warm_p_next = W->warm_p[nxt];
-        a.warm_s_next = W->warm_s[nxt];
-        a.warm_n_next = W->warm_n[nxt];
-        k_batched_step<BLOCK, true, ISL><<<grid, BLOCK, lds, cs>>>(a);
-        k_zero_i32<<<1, 64, 0, cs>>>(a.queue, 2);  // counter buffer A is zero between launches
-        NANS_HIP(hipGetLastError());
-        W->warm_flip = nxt;
-    }
-    W->graph_block = BLOCK;
-    W->graph_grid = grid;
-    W->graph_lds = (int)lds;
-    W->graph_wave = sp.bodies;
-    W->graph_nwave = sp.nwave;
-    return NANS_OK;
-}
-
-int batched_run_warm(nans_ctx *ctx, int nsteps, int block)
-{
-    nans_worlds *W = ctx->worlds;
-    NANS_REQUIRE(W->nmax <= BATCH_MAX_BODIES, NANS_ERR_CAPACITY,
-                 "the batched step keeps a world in LDS: at most %d bodies per world (largest: %d)",
-                 BATCH_MAX_BODIES, W->nmax);
-    hipStream_t cs = ctx->own_stream;
-    if (!W->ev_in) {
-        NANS_HIP(hipEventCreateWithFlags(&W->ev_in, hipEventDisableTiming));
-        NANS_HIP(hipEventCreateWithFlags(&W->ev_out, hipEventDisableTiming));
-        NANS_HIP(hipEventCreate(&W->ev_t0));
-        NANS_HIP(hipEventCreate(&W->ev_t1));
-    }
-    NANS_TRY(warm_prepare(ctx));
-    NANS_TRY(setup_floor(ctx, ctx->stream));
-    drop_graph(W);  // the graph_* launch shape below describes these launches
-    NANS_HIP(hipEventRecord(W->ev_in, ctx->stream));
-    NANS_HIP(hipStreamWaitEvent(cs, W->ev_in, 0));
-    NANS_HIP(hipEventRecord(W->ev_t0, cs));
+    if (ctx->warm) NANS_TRY(warm_prepare(ctx));
+    NANS_TRY(setup_floor(ctx, s));
+    NANS_HIP(hipEventRecord(W->ev_t0, s));
     NANS_TRY(by_shape(block, ctx->p.fp64_islands != 0, [&](auto B, auto I) {
-        return batched_warm_launches<decltype(B)::value, decltype(I)::value>(ctx, nsteps, cs);
+        constexpr int BL = decltype(B)::value;
+        constexpr bool IS = decltype(I)::value;
+        return ctx->warm ? batched_launches<BL, true, IS>(ctx, nsteps, s, nullptr)
+                         : batched_launches<BL, false, IS>(ctx, nsteps, s, nullptr);
     }));
-    NANS_HIP(hipEventRecord(W->ev_t1, cs));
-    NANS_HIP(hipEventRecord(W->ev_out, cs));
-    NANS_HIP(hipStreamWaitEvent(ctx->stream, W->ev_out, 0));
+    NANS_HIP(hipEventRecord(W->ev_t1, s));
     W->timed_steps = nsteps;
     return NANS_OK;
 }
@@ -1980,35 +1916,23 @@ int batched_block(nans_ctx *ctx)
     return W->nmax <= 64 ? 128 : 256;
 }
 
-template <int BLOCK, bool ISL>
-static int batched_recorded_launch(nans_ctx *ctx, hipStream_t s, ContactRec *rec_out, const int64_t *rec_off,
-                                   int *rec_count, const int *rec_cap)
-{
-    BatchArgsT<false> a;
-    int grid = 0;
-    size_t lds = 0;
-    NANS_TRY((batched_prepare<BLOCK, false, ISL>(ctx, a, &grid, &lds)));
-    a.rec_out = rec_out;
-    a.rec_off = rec_off;
-    a.rec_count = rec_count;
-    a.rec_cap = rec_cap;
-    k_batched_step<BLOCK, false, ISL><<<grid, BLOCK, lds, s>>>(a);
-    k_zero_i32<<<1, 64, 0, s>>>(a.queue, 2);  // counter buffer A is zero between launches
-    NANS_HIP(hipGetLastError());
-    return NANS_OK;
-}
-
-int batched_step_recorded(nans_ctx *ctx, hipStream_t s, ContactRec *rec_out, const int64_t *rec_off, int *rec_count,
-                          const int *rec_cap)
+int batched_run_recorded(nans_ctx *ctx, int nsteps, hipStream_t s, const BatchRecord &rec)
 {
     nans_worlds *W = ctx->worlds;
     NANS_REQUIRE(W->nmax <= BATCH_MAX_BODIES, NANS_ERR_CAPACITY,
                  "the batched step keeps a world in LDS: at most %d bodies per world (largest: %d)",
                  BATCH_MAX_BODIES, W->nmax);
-    return by_shape(batched_block(ctx), ctx->p.fp64_islands != 0, [&](auto B, auto I) {
-        return batched_recorded_launch<decltype(B)::value, decltype(I)::value>(ctx, s, rec_out, rec_off, rec_count,
-                                                                              rec_cap);
-    });
+    for (int done = 0; done < nsteps; done += BATCH_LAUNCH_STEPS) {
+        BatchRecord r = rec;
+        r.state += (int64_t)done * STATE_FIELDS * W->N;
+        r.rec += done * rec.rec_stride;
+        r.rec_count += (int64_t)done * W->nworlds;
+        NANS_TRY(by_shape(batched_block(ctx), ctx->p.fp64_islands != 0, [&](auto B, auto I) {
+            return batched_launches<decltype(B)::value, false, decltype(I)::value>(
+                ctx, std::min(nsteps - done, BATCH_LAUNCH_STEPS), s, &r);
+        }));
+    }
+    return NANS_OK;
 }
 
 }  // namespace nans
@@ -2024,8 +1948,7 @@ int nans_step_batched(nans_ctx *ctx, int32_t nsteps)
     nans_worlds *W = ctx->worlds;
     int block = batched_block(ctx);
     NANS_TRY(snapshot_take(ctx, ctx->stream));
-    if (ctx->warm) NANS_TRY(batched_run_warm(ctx, nsteps, block));
-    else NANS_TRY(batched_run(ctx, nsteps, block));
+    NANS_TRY(batched_run(ctx, nsteps, block));
     NANS_HIP(hipStreamSynchronize(ctx->stream));
     float ms = 0.0f;
     NANS_HIP(hipEventElapsedTime(&ms, W->ev_t0, W->ev_t1));
@@ -2041,11 +1964,11 @@ int nans_batched_timing(nans_ctx *ctx, nans_timing *t)
     NANS_REQUIRE(W->timed_steps > 0, NANS_ERR_STATE, "no batched step has run");
     t->steps = W->timed_steps;
     t->elapsed_ms = W->timed_ms;
-    t->threads_per_world = W->graph_block;
-    t->workgroups = W->graph_grid;
-    t->lds_bytes = W->graph_lds;
-    t->wave_world_bodies = W->graph_wave;
-    t->wave_worlds = W->graph_nwave;
+    t->threads_per_world = W->shape_block;
+    t->workgroups = W->shape_grid;
+    t->lds_bytes = W->shape_lds;
+    t->wave_world_bodies = W->shape_wave;
+    t->wave_worlds = W->shape_nwave;
     return NANS_OK;
 }
 
@@ -2121,7 +2044,7 @@ int nans_autotune_batched(nans_ctx *ctx, int32_t nsteps, nans_tuning *out)
             prev_nbig = sp.nbig;
             W->tuned_wave = bounds[b];
             float ms = -1.0f;
-            // one untimed step captures the graph; then nsteps timed steps
+            // one untimed step (scratch); then nsteps timed steps
             int r = batched_run(ctx, 1, cand[c]);
             if (r == NANS_OK) r = batched_run(ctx, nsteps, cand[c]);
             if (r == NANS_OK) {
