@@ -70,12 +70,11 @@ __host__ __device__ inline V3 rk4_adjoint(float dt, V3 y0, V3 F, float m, const 
     return gy0;
 }
 
-// Forward values Constraint read for one contact.
-struct ContactBodies {
-    V3 PA, PB;          // positions (PB: the floor's centre for floor pairs)
-    V3 V1, W1, V2, W2;  // velocities when the contact was applied (floor: zero)
-    float mA, IA, mB, IB;
-    bool two_sided;     // B is a body (its velocities are written)
+// Velocities Constraint read for one contact (floor: zero), and whether B is a body
+// (its velocities are written).
+struct ContactVel {
+    V3 V1, W1, V2, W2;
+    bool two_sided;
 };
 
 // Adjoints of one contact: gV*/gW* hold the adjoints of the velocities after the
@@ -86,45 +85,51 @@ struct ContactGrad {
     float gmA, gIA, gmB, gIB, gCf, gCr;
 };
 
-__host__ __device__ inline void constraint_adjoint(const ContactRec &c, const ContactBodies &b, const StepConsts &k,
-                                                   float Cf, float Cr, ContactGrad &g)
-{
-    // ---- forward values, as constraint() computes them
-    V3 N = normalize(mk3(c.n[0], c.n[1], c.n[2]));
-    if (veq(N, mk3(0.0f, 0.0f, 0.0f))) N = normalize(sub(b.PB, b.PA));
-    const V3 R1 = sub(mk3(c.pa[0], c.pa[1], c.pa[2]), b.PA);
-    const V3 R2 = sub(mk3(c.pb[0], c.pb[1], c.pb[2]), b.PB);
-    const V3 T1 = N.x >= 0.57735f ? mk3(N.y, -N.x, 0.0f) : mk3(0.0f, N.z, -N.y);
-    const V3 T2 = cross(N, T1);
-    const float Depth = dot(sub(add(b.PA, R1), add(b.PB, R2)), N);
-    const float InvI1 = 1.0f / b.IA, InvI2 = 1.0f / b.IB;
-    const float InvM1 = 1.0f / b.mA, InvM2 = 1.0f / b.mB;
-    const V3 RN1 = cross(R1, N), RN2 = cross(R2, N);
-    const V3 R1T1 = cross(R1, T1), R2T1 = cross(R2, T1), R1T2 = cross(R1, T2), R2T2 = cross(R2, T2);
-    const float qn1 = dot(RN1, RN1), qn2 = dot(RN2, RN2);
-    const float q11 = dot(R1T1, R1T1), q21 = dot(R2T1, R2T1), q12 = dot(R1T2, R1T2), q22 = dot(R2T2, R2T2);
-    const float JMJn = 1.0f / ((InvM1 + InvM2) + (InvI1 * qn1 - InvI2 * qn2));
-    const float JMJt1 = 1.0f / ((InvM1 + InvM2) + (InvI1 * q11 - InvI2 * q21));
-    const float JMJt2 = 1.0f / ((InvM1 + InvM2) + (InvI1 * q12 - InvI2 * q22));
-    const float JdVn = dot(sub(sub(add(b.V1, cross(b.W1, N)), b.V2), cross(b.W2, N)), N);
-    const float JdVt1 = dot(sub(sub(add(b.V1, cross(b.W1, T1)), b.V2), cross(b.W2, T1)), T1);
-    const float JdVt2 = dot(sub(sub(add(b.V1, cross(b.W1, T2)), b.V2), cross(b.W2, T2)), T2);
-    const float kb = -k.beta / k.dt;
-    const float Bb = kb * Depth + Cr * JdVn;
-    const float L = (-JdVn + Bb) * JMJn;
-    const float LT1 = (-JdVt1) * JMJt1;
-    const float LT2 = (-JdVt2) * JMJt2;
+// What the reverse of one contact needs beside its position-only terms and the
+// adjoints of the velocities after it: it depends on the velocities the contact
+// read, so it is made once they are known, for all contacts at once.
+struct ContactReplay {
+    float JdVn, JdVt1, JdVt2, Bb;
+    float dln, dlt1, dlt2;
+};
 
-    // ---- replay of the iterations: sumN after each, and the clamps taken
-    //      code bit 0: sumN clamped to 0; bits 1-2 / 3-4: tangent 1 / 2 set to
-    //      -MaxLT (1) or +MaxLT (2)
-    const int K = k.solver_iterations < ADJ_MAX_ITERS ? k.solver_iterations : ADJ_MAX_ITERS;
-    float shist[ADJ_MAX_ITERS];
-    unsigned char code[ADJ_MAX_ITERS];
+// Impulse iterations: sumN after each, and the clamps taken.  code bit 0: sumN
+// clamped to 0; bits 1-2 / 3-4: tangent 1 / 2 set to -MaxLT (1) or +MaxLT (2).
+struct LocalHistory {
+    float s[ADJ_MAX_ITERS];
+    unsigned char c[ADJ_MAX_ITERS];
+    __host__ __device__ void put(int it, float sum, int code)
+    {
+        s[it] = sum;
+        c[it] = (unsigned char)code;
+    }
+    __host__ __device__ float sum(int it) const { return s[it]; }
+    __host__ __device__ int code(int it) const { return c[it]; }
+};
+
+__host__ __device__ inline int adj_iterations(const StepConsts &k)
+{
+    return k.solver_iterations < ADJ_MAX_ITERS ? k.solver_iterations : ADJ_MAX_ITERS;
+}
+
+// Forward values as contact_apply() computes them, and the replay of its iterations
+// into h.
+template <class History>
+__host__ __device__ inline void contact_replay(const ContactTerms &t, const ContactVel &b, const StepConsts &k,
+                                               float Cf, float Cr, ContactReplay &p, History &h)
+{
+    p.JdVn = dot(sub(sub(add(b.V1, cross(b.W1, t.N)), b.V2), cross(b.W2, t.N)), t.N);
+    p.JdVt1 = dot(sub(sub(add(b.V1, cross(b.W1, t.T1)), b.V2), cross(b.W2, t.T1)), t.T1);
+    p.JdVt2 = dot(sub(sub(add(b.V1, cross(b.W1, t.T2)), b.V2), cross(b.W2, t.T2)), t.T2);
+    p.Bb = t.bdepth + Cr * p.JdVn;
+    const float L = (-p.JdVn + p.Bb) * t.JMJn;
+    const float LT1 = (-p.JdVt1) * t.JMJt1;
+    const float LT2 = (-p.JdVt2) * t.JMJt2;
+    const int K = adj_iterations(k);
     const double cf2 = 1.4142135623730951 * (double)Cf;
     float sumN = 0.0f, sumT1 = 0.0f, sumT2 = 0.0f, dln = 0.0f, dlt1 = 0.0f, dlt2 = 0.0f;
     for (int it = 0; it < K; ++it) {
-        unsigned char cd = 0;
+        int cd = 0;
         const float old = sumN;
         sumN += L;
         if (sumN < 0.0f) {
@@ -145,9 +150,26 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
         if (sumT2 < -M) { sumT2 = -M; t2 = 1; }
         if (sumT2 > M) { sumT2 = M; t2 = 2; }
         dlt2 = sumT2 - o2;
-        shist[it] = sumN;
-        code[it] = (unsigned char)(cd | (t1 << 1) | (t2 << 3));
+        h.put(it, sumN, cd | (t1 << 1) | (t2 << 3));
     }
+    p.dln = dln;
+    p.dlt1 = dlt1;
+    p.dlt2 = dlt2;
+}
+
+template <class History>
+__host__ __device__ inline void constraint_adjoint(const ContactTerms &t, const ContactReplay &p, bool two_sided,
+                                                   const StepConsts &k, float Cf, float Cr, const History &h,
+                                                   ContactGrad &g)
+{
+    const V3 N = t.N, T1 = t.T1, T2 = t.T2;
+    const V3 RN1 = t.RN1, RN2 = t.RN2, R1T1 = t.R1T1, R2T1 = t.R2T1, R1T2 = t.R1T2, R2T2 = t.R2T2;
+    const float InvM1 = t.InvM1, InvM2 = t.InvM2, InvI1 = t.InvI1, InvI2 = t.InvI2;
+    const float dln = p.dln, dlt1 = p.dlt1, dlt2 = p.dlt2;
+    const float qn1 = dot(RN1, RN1), qn2 = dot(RN2, RN2);
+    const float q11 = dot(R1T1, R1T1), q21 = dot(R2T1, R2T1), q12 = dot(R1T2, R1T2), q22 = dot(R2T2, R2T2);
+    const float kb = -k.beta / k.dt;
+    const double cf2 = 1.4142135623730951 * (double)Cf;
 
     // ---- reverse of the impulse application
     const V3 lin = add(add(mul(N, dln), mul(T1, dlt1)), mul(T2, dlt2));
@@ -157,7 +179,7 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
     float gInvM1 = dot(lin, g.gV1);
     float gInvI1 = dot(add(add(mul(RN1, dln), mul(R1T1, dlt1)), mul(R1T2, dlt2)), g.gW1);
     float gInvM2 = 0.0f, gInvI2 = 0.0f;
-    if (b.two_sided) {
+    if (two_sided) {
         gdln -= InvM2 * dot(N, g.gV2) + InvI2 * dot(RN2, g.gW2);
         gdlt1 -= InvM2 * dot(T1, g.gV2) + InvI2 * dot(R2T1, g.gW2);
         gdlt2 -= InvM2 * dot(T2, g.gV2) + InvI2 * dot(R2T2, g.gW2);
@@ -166,12 +188,13 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
     }
 
     // ---- reverse of the iterations (only the last one's deltas are outputs)
+    const int K = adj_iterations(k);
     float gs = 0.0f, gt1 = 0.0f, gt2 = 0.0f;
     float gL = 0.0f, gLT1 = 0.0f, gLT2 = 0.0f, gCf = 0.0f;
     for (int it = K - 1; it >= 0; --it) {
         const bool last = it == K - 1;
-        const int cd = code[it];
-        const float sn = shist[it];
+        const int cd = h.code(it);
+        const float sn = h.sum(it);
         float gM = 0.0f;
         // tangent 2: t' = clamp(t + LT2), dlt2 = t' - t
         {
@@ -204,16 +227,16 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
     }
 
     // ---- reverse of the impulse terms
-    const float gJMJn = (-JdVn + Bb) * gL;
-    const float gBb = JMJn * gL;
-    const float gJdVn = -JMJn * gL + Cr * gBb;
+    const float gJMJn = (-p.JdVn + p.Bb) * gL;
+    const float gBb = t.JMJn * gL;
+    const float gJdVn = -t.JMJn * gL + Cr * gBb;
     const float gDepth = kb * gBb;
-    const float gCr = JdVn * gBb;
-    const float gJdVt1 = -JMJt1 * gLT1, gJMJt1 = -JdVt1 * gLT1;
-    const float gJdVt2 = -JMJt2 * gLT2, gJMJt2 = -JdVt2 * gLT2;
-    const float gDn = -JMJn * JMJn * gJMJn;
-    const float gDt1 = -JMJt1 * JMJt1 * gJMJt1;
-    const float gDt2 = -JMJt2 * JMJt2 * gJMJt2;
+    const float gCr = p.JdVn * gBb;
+    const float gJdVt1 = -t.JMJt1 * gLT1, gJMJt1 = -p.JdVt1 * gLT1;
+    const float gJdVt2 = -t.JMJt2 * gLT2, gJMJt2 = -p.JdVt2 * gLT2;
+    const float gDn = -t.JMJn * t.JMJn * gJMJn;
+    const float gDt1 = -t.JMJt1 * t.JMJt1 * gJMJt1;
+    const float gDt2 = -t.JMJt2 * t.JMJt2 * gJMJt2;
     gInvM1 += gDn + gDt1 + gDt2;
     gInvM2 += gDn + gDt1 + gDt2;
     gInvI1 += qn1 * gDn + q11 * gDt1 + q12 * gDt2;
@@ -223,7 +246,7 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
     const V3 gdw = add(add(cross(N, mul(N, gJdVn)), cross(T1, mul(T1, gJdVt1))), cross(T2, mul(T2, gJdVt2)));
     g.gV1 = add(g.gV1, gdv);
     g.gW1 = add(g.gW1, gdw);
-    if (b.two_sided) {
+    if (two_sided) {
         g.gV2 = sub(g.gV2, gdv);
         g.gW2 = sub(g.gW2, gdw);
     }
@@ -231,15 +254,15 @@ __host__ __device__ inline void constraint_adjoint(const ContactRec &c, const Co
     g.gPB = mul(N, -gDepth);
     g.gmA = -InvM1 * InvM1 * gInvM1;
     g.gIA = -InvI1 * InvI1 * gInvI1;
-    g.gmB = b.two_sided ? -InvM2 * InvM2 * gInvM2 : 0.0f;
-    g.gIB = b.two_sided ? -InvI2 * InvI2 * gInvI2 : 0.0f;
+    g.gmB = two_sided ? -InvM2 * InvM2 * gInvM2 : 0.0f;
+    g.gIB = two_sided ? -InvI2 * InvI2 * gInvI2 : 0.0f;
     g.gCf = gCf;
     g.gCr = gCr;
 }
 
-// Per-contact record of the adjoint kernel: the velocities Constraint read, the
-// dependency round the contact was applied in, and its friction/restitution
-// adjoints (summed per world in contact order afterwards).
+// Record of a contact that no thread of the adjoint kernel holds in registers: the
+// velocities Constraint read, the dependency round the contact was applied in, and
+// its friction/restitution adjoints (summed per world in contact order afterwards).
 struct AdjTape {
     float v1[3], w1[3], v2[3], w2[3];
     int round;
