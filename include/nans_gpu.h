@@ -319,7 +319,9 @@ int nans_reset_stats(nans_ctx *ctx);
  *
  * nans_rollout advances every world by nsteps batched steps from the current
  * state, as nans_step_batched does, and keeps the state (pos, vel, angvel,
- * angles, force, torque) every checkpoint_every steps on the device.
+ * angles, force, torque) and the contacts of every step on the device while that
+ * takes at most 8 GiB and a quarter of the free memory, else the state every
+ * checkpoint_every steps (also where the batch records its contacts).
  *
  * nans_adjoint returns the gradient of a loss L(final state) with respect to the
  * initial state and the per-body mass and moment of inertia and the per-world
@@ -328,8 +330,8 @@ int nans_reset_stats(nans_ctx *ctx);
  * impulse iterations (code/nans.cpp:1020-1329) and of IntegrateVelocities
  * (code/nans.cpp:1331-1349); the GJK/EPA outcome -- which pairs touch, in which
  * order, with which normal and lever arms PointA - PosA, PointB - PosB -- is held
- * fixed at the rollout's.  The segments between checkpoints are recomputed on the
- * device.  The mass gradient counts mass only: when the moment of inertia is a
+ * fixed at the rollout's.  Where only checkpoints were kept, the segments between
+ * them are recomputed on the device.  The mass gradient counts mass only: when the moment of inertia is a
  * function of the mass, add dl_moi * d(moi)/d(mass).  The batch is left at the
  * rollout's final state.  Arrays are host memory: vectors [3][N] planes, dl_mass
  * and dl_moi [N], dl_friction and dl_restitution [nworlds]; NULL inputs count as

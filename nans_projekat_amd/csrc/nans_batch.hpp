@@ -69,6 +69,9 @@ struct BatchArgs {
     const int64_t *rec_off; // rec_count[k * rec_count_stride + w]
     int *rec_count;
     int rec_count_stride;
+    unsigned long long *rec_pos;  // or, if set, the lists one after another as they come:
+    int *rec_start;               // step k's of world w at rec_start[k * rec_count_stride + w],
+    int rec_total;                // rec_total records in all (those beyond are only counted)
     const int *rec_cap;
     unsigned long long *cnt;
 };
@@ -124,6 +127,10 @@ struct BatchRecord {
     const int64_t *rec_off;
     int *rec_count;  // nworlds per step
     const int *rec_cap;
+    // set: lists one after another instead, rec_total records of room
+    unsigned long long *pos = nullptr;
+    int *start = nullptr;  // nworlds per step
+    int rec_total = 0;
 };
 int batched_run_recorded(nans_ctx *ctx, int nsteps, hipStream_t s, const BatchRecord &rec);
 

@@ -886,10 +886,27 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
         }
     }
     if (a.rec_out) {
-        ContactRec *dst = a.rec_out + step * a.rec_stride + a.rec_off[w];
-        int rc = a.rec_cap[w];
-        for (int c = tid; c < ncon && c < rc; c += T) dst[c] = con[c];
-        if (tid == 0) a.rec_count[(int64_t)step * a.rec_count_stride + w] = ncon;
+        const int64_t k = (int64_t)step * a.rec_count_stride + w;
+        if (tid == 0) a.rec_count[k] = ncon;
+        if (a.rec_pos) {  // the next ncon records, while there are as many
+            int off = 0;
+            if (tid == 0) a.rec_start[k] = off = (int)min(atomicAdd(a.rec_pos, (unsigned long long)ncon),
+                                                          (unsigned long long)a.rec_total);
+            if (t.whole) {
+                if (tid == 0) wave_tot[0] = off;
+                __syncthreads();
+                off = wave_tot[0];
+            } else {
+                off = __builtin_amdgcn_readfirstlane(off);
+            }
+            ContactRec *dst = a.rec_out + off;
+            const int room = a.rec_total - off;
+            for (int c = tid; c < ncon && c < room; c += T) dst[c] = con[c];
+        } else {
+            ContactRec *dst = a.rec_out + step * a.rec_stride + a.rec_off[w];
+            const int rc = a.rec_cap[w];
+            for (int c = tid; c < ncon && c < rc; c += T) dst[c] = con[c];
+        }
     }
     t.sync();
 }
@@ -1824,6 +1841,9 @@ static int batched_prepare(nans_ctx *ctx, BatchArgs &a, int *grid_out, size_t *l
     a.rec_count = W->rec_count;
     a.rec_count_stride = 0;
     a.rec_cap = W->rec_cap;
+    a.rec_pos = nullptr;
+    a.rec_start = nullptr;
+    a.rec_total = 0;
     a.cnt = W->cnt;
     W->shape_block = BLOCK;
     W->shape_grid = grid;
@@ -1857,6 +1877,9 @@ static int batched_launches(nans_ctx *ctx, int nsteps, hipStream_t s, const Batc
         a.rec_count = rec->rec_count;
         a.rec_count_stride = W->nworlds;
         a.rec_cap = rec->rec_cap;
+        a.rec_pos = rec->pos;
+        a.rec_start = rec->start;
+        a.rec_total = rec->rec_total;
     }
     if constexpr (WARM) {
         a.warm_p0 = W->warm_p[0];
@@ -1927,6 +1950,7 @@ int batched_run_recorded(nans_ctx *ctx, int nsteps, hipStream_t s, const BatchRe
         r.state += (int64_t)done * STATE_FIELDS * W->N;
         r.rec += done * rec.rec_stride;
         r.rec_count += (int64_t)done * W->nworlds;
+        if (r.start) r.start += (int64_t)done * W->nworlds;
         NANS_TRY(by_shape(batched_block(ctx), ctx->p.fp64_islands != 0, [&](auto B, auto I) {
             return batched_launches<decltype(B)::value, false, decltype(I)::value>(
                 ctx, std::min(nsteps - done, BATCH_LAUNCH_STEPS), s, &r);

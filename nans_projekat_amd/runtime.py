@@ -348,8 +348,9 @@ class Context:
 
     # ------------------------------------------------------------------ differentiable rollout
     def rollout(self, nsteps: int, checkpoint_every: int = 16) -> None:
-        """nsteps batched steps from the current state, keeping the state every
-        checkpoint_every steps for adjoint()."""
+        """nsteps batched steps from the current state, keeping what adjoint() needs:
+        every step, or where that takes too much memory the state every
+        checkpoint_every steps."""
         self._sync_stream()
         check(self.lib.nans_rollout(self.h, int(nsteps), int(checkpoint_every)))
 
