@@ -16,10 +16,15 @@ constexpr int BATCH_MAX_BODIES = 512;    // bodies of one world kept in LDS by t
 constexpr int SCAN_THREADS = 1024;
 constexpr int SOLVE_THREADS = 1024;
 // The plain step's solve for worlds of at most PLAIN_SMALL_BODIES bodies: 256
-// threads, and the terms of the first PLAIN_SMALL_TERMS contacts kept in LDS.
+// threads, with lists, bodies and as many contact terms as a CU's LDS holds.
 constexpr int PLAIN_SMALL_THREADS = 256;
 constexpr int PLAIN_SMALL_BODIES = 512;
-constexpr int PLAIN_SMALL_TERMS = 320;
+constexpr size_t PLAIN_SMALL_LDS = 156 * 1024;
+// head[], two counters, list[2 n], body planes
+constexpr size_t plain_small_fixed_bytes(int n)
+{
+    return sizeof(int) * ((size_t)(3 + F_NLDS) * ((n + 3) & ~3) + 4);
+}
 constexpr int CULL_CHUNK = 4096;          // canonical pairs per block of the plain cull
 
 enum : int {

@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstddef>
 #include <cmath>
 #include <map>
 #include <numeric>
@@ -188,46 +189,258 @@ struct WorldSrc {
     }
 };
 
-// Dependency rounds of SolveConstraints over con[0..ncon) (see the file comment).
-// head[] has room for n ints; done[] for ncon.  The body slots of each thread's
-// first REG contacts stay in registers for all rounds; contacts beyond REG * BLOCK
-// are read from con[] each round.  The plain step's solve keeps SOLVE_REG; the
-// batched step, compiled for three waves per SIMD, keeps one (two cost it 2.5 %
-// of its step in spilled registers).
-constexpr int SOLVE_REG = 2;
-constexpr int BATCH_SOLVE_REG = 1;
-
 // Contact c of a world's ordered list.
 struct DirectCon {
     ContactRec *p;
     __device__ ContactRec &operator()(int c) const { return p[c]; }
 };
 
-// Room for Constraint's position-only terms of the first contacts: two
-// segments of LDS that are idle during SolveConstraints (terms of contact c in
-// a[c] for c < na, else in b[c - na] for c < na + nb).
-struct PreTerms {
-    ContactTerms *a = nullptr;
-    int na = 0;
-    ContactTerms *b = nullptr;
-    int nb = 0;
-    __device__ ContactTerms &operator()(int c) const { return c < na ? a[c] : b[c - na]; }
+// Value of lane U of the quad in its four lanes (all active).
+template <int U>
+__device__ __forceinline__ float quad_bcast(float v)
+{
+    return dpp_f<U * 0x55>(v);
+}
+
+// contact_apply by the four lanes of a quad: lane 0, 1, 2 works out the impulse along
+// N, T1, T2 and then component x, y, z of the bodies' velocities (lane 3 follows lane
+// 0 and stores nothing).  Every expression is contact_apply's, so are the results; a
+// contact takes 230 instructions of a wave instead of 600, and 16 fit a wave.
+// t: the lane's part of the contact's terms (quad_terms); sums: its accumulators (warm start) or
+// null; dl: receives dln, dlt1, dlt2, or null.
+static_assert(sizeof(ContactTerms) == 35 * sizeof(float) && offsetof(ContactTerms, RN1) == 9 * sizeof(float) &&
+                  offsetof(ContactTerms, JMJn) == 27 * sizeof(float) &&
+                  offsetof(ContactTerms, bdepth) == 30 * sizeof(float) &&
+                  offsetof(ContactTerms, InvI2) == 34 * sizeof(float),
+              "quad_terms reads the terms by position");
+struct QuadTerms {
+    V3 D;                // this lane's direction
+    float JMJ, bdepth;   // and its 1 / (J M^-1 J^T); -beta / dt * Depth
+    float g[9];          // component of N T1 T2 RN1 RN2 R1T1 R2T1 R1T2 R2T2
+    float InvM1, InvM2, InvI1, InvI2;
 };
 
-// pre receives the terms of the first contacts in one parallel pass (as many as
-// it holds), so that the rounds only evaluate the velocity-dependent part for
-// them.  con(c) is contact c's record (DirectCon).
-template <bool WARM = false, int REG = SOLVE_REG, class Con>
+__device__ __forceinline__ QuadTerms quad_terms(const ContactTerms *t)
+{
+    const int q = (int)(threadIdx.x & 3), e = q == 3 ? 0 : q;
+    const float *f = reinterpret_cast<const float *>(t);
+    QuadTerms o;
+    o.D = mk3(f[3 * e], f[3 * e + 1], f[3 * e + 2]);
+    o.JMJ = f[27 + e];
+    o.bdepth = f[30];
+#pragma unroll
+    for (int j = 0; j < 9; ++j) o.g[j] = f[3 * j + e];
+    o.InvM1 = f[31];
+    o.InvM2 = f[32];
+    o.InvI1 = f[33];
+    o.InvI2 = f[34];
+    return o;
+}
+
+template <bool WARM>
+__device__ __forceinline__ void quad_apply(const Planes &B, int sa, int sb, const QuadTerms &t, const StepConsts &k,
+                                           float Cf, float Cr, float *sums, float *dl)
+{
+    const int q = (int)(threadIdx.x & 3);
+    const int e = q == 3 ? 0 : q;  // direction, then component
+    const V3 zero = mk3(0.0f, 0.0f, 0.0f);
+    const V3 V1 = B.get3(F_VX, sa), W1 = B.get3(F_WX, sa);
+    V3 V2 = zero, W2 = zero;
+    if (sb >= 0) {
+        V2 = B.get3(F_VX, sb);
+        W2 = B.get3(F_WX, sb);
+    }
+    float sum = 0.0f;  // this lane's accumulator
+    if constexpr (WARM) sum = sums[e];
+
+    const V3 dV = sub(sub(add(V1, cross(W1, t.D)), V2), cross(W2, t.D));
+    const float J = dot(dV, t.D);
+    const float Bb = t.bdepth + Cr * J;
+    const float Lambda = (e == 0 ? -J + Bb : -J) * t.JMJ;
+    const float LambdaN = quad_bcast<0>(Lambda);
+    float sumN = quad_bcast<0>(sum), last = 0.0f;
+    const double cf_sqrt2 = 1.4142135623730951 * (double)Cf;
+    auto iterate = [&]() {
+        sumN += LambdaN;
+        if (sumN < 0.0f) sumN = 0.0f;
+        const float MaxLT = (float)(cf_sqrt2 * (double)sumN);
+        sum += Lambda;
+        if (sum < -MaxLT) sum = -MaxLT;
+        if (sum > MaxLT) sum = MaxLT;
+    };
+    if (k.solver_iterations > 0) {
+        if (k.solver_iterations == 10) {
+#pragma unroll
+            for (int it = 1; it < 10; ++it) iterate();
+        } else {
+#pragma unroll 4
+            for (int it = 1; it < k.solver_iterations; ++it) iterate();
+        }
+        const float oldN = sumN, old = sum;
+        iterate();
+        last = e == 0 ? sumN - oldN : sum - old;
+    }
+    const float dln = quad_bcast<0>(last), dlt1 = quad_bcast<1>(last), dlt2 = quad_bcast<2>(last);
+    auto comp = [&](V3 v) { return e == 0 ? v.x : (e == 1 ? v.y : v.z); };
+    const float LinN = t.g[0] * dln, LinT1 = t.g[1] * dlt1, LinT2 = t.g[2] * dlt2;
+    float va = comp(V1), wa = comp(W1), vb = comp(V2), wb = comp(W2);
+    va = va + LinN * t.InvM1;
+    vb = vb - LinN * t.InvM2;
+    wa = wa + t.g[3] * dln * t.InvI1;
+    wb = wb - t.g[4] * dln * t.InvI2;
+    va = va + LinT1 * t.InvM1;
+    vb = vb - LinT1 * t.InvM2;
+    wa = wa + t.g[5] * dlt1 * t.InvI1;
+    wb = wb - t.g[6] * dlt1 * t.InvI2;
+    va = va + LinT2 * t.InvM1;
+    vb = vb - LinT2 * t.InvM2;
+    wa = wa + t.g[7] * dlt2 * t.InvI1;
+    wb = wb - t.g[8] * dlt2 * t.InvI2;
+    if (q < 3) {
+        B.at(F_VX + q, sa) = va;
+        B.at(F_WX + q, sa) = wa;
+        if (sb >= 0) {  // the floor's velocities are never written (code/nans.cpp:1280-1289)
+            B.at(F_VX + q, sb) = vb;
+            B.at(F_WX + q, sb) = wb;
+        }
+        if constexpr (WARM) sums[q] = q == 0 ? sumN : sum;
+        if (dl) dl[q] = last;
+    }
+}
+
+// Where a team keeps the position-only terms of its contacts: one segment of LDS, or
+// two, then one of global memory.
+struct LdsTerms {
+    ContactTerms *a;
+    int na;
+    __device__ int room() const { return na; }
+    __device__ void put(int c, const ContactTerms &o) const { a[c] = o; }
+    __device__ QuadTerms quad(int c) const { return quad_terms(a + c); }
+};
+
+struct SplitTerms {
+    ContactTerms *a, *b, *g;
+    int na, nb, ng;
+    __device__ int room() const { return na + nb + ng; }
+    __device__ void put(int c, const ContactTerms &o) const
+    {
+        if (c < na + nb) *(c < na ? a + c : b + (c - na)) = o;
+        else g[c - na - nb] = o;
+    }
+    __device__ QuadTerms quad(int c) const
+    {
+        if (c < na + nb) return quad_terms(c < na ? a + c : b + (c - na));
+        return quad_terms(g + (c - na - nb));
+    }
+};
+
+// Dependency rounds of SolveConstraints over con[0..ncon) (see the file comment) for
+// a world of n <= 32767 bodies.  head[] has room for n ints, list[] for 2 n; done[]
+// for ncon.  First the terms of every contact in one parallel pass; should they not
+// fit the store, the list is solved in parts, one after another, which keeps its order.
+// In a round every thread looks whether its pending contacts are the earliest of their
+// bodies and lists those that are; then quads apply the listed contacts.  A round
+// readies few contacts (some tens of a world's hundreds), which a contact per lane
+// spread over the team's waves, each running the whole arithmetic for a few lanes, and
+// bounds a step by its latency: the plain step of a 181-body world 221 -> 170 us, 601
+// worlds with warm start 34.3 -> 31.5 ms per 30 steps, 4096 worlds, bound by the
+// narrowphase's instructions, 81.0 -> 81.0 ms per 60.
+// The bodies of each thread's first REG contacts of a part stay in registers.  Two
+// barriers a round: the next round's keys may start while quads still apply.
+constexpr int SOLVE_REG = 4;
+
+template <bool WARM, int REG, class Con, class Terms>
+__device__ __forceinline__ void solve_packed(const Team &t, const Planes &B, int n, const Con &con, int ncon, int *done,
+                                    int *head, int *list, int *count, const Terms &ts, const FloorDev &fl,
+                                    const StepConsts &k, float Cf, float Cr, float *warm, bool keep_dl)
+{
+    const int tid = t.rank, T = t.size;
+    unsigned *hk = reinterpret_cast<unsigned *>(head);
+    for (int base = 0; base < ncon; base += ts.room()) {
+        const int m = min(ncon - base, ts.room());
+        // terms and bodies; heads and counters of the rounds
+        int slots[REG];
+        for (int c = tid; c < m; c += T) {
+            ContactTerms o;
+            contact_terms(B, con(base + c), fl, k, o);
+            ts.put(c, o);
+        }
+        auto pack = [&](int c) {
+            const ContactRec &r = con(base + c);
+            return (int)((unsigned)r.slot_a | ((unsigned)r.slot_b << 16));  // negative: the floor
+        };
+#pragma unroll
+        for (int r = 0; r < REG; ++r) slots[r] = tid + r * T < m ? pack(tid + r * T) : 0;
+        unsigned pend = 0;  // bit r: contact tid + r T is pending
+#pragma unroll
+        for (int r = 0; r < REG; ++r) pend |= tid + r * T < m ? 1u << r : 0u;
+        for (int c = tid + REG * T; c < m; c += T) done[c] = 0;
+        for (int i = tid; i < n; i += T) hk[i] = 0u;
+        if (tid < 2) count[tid] = 0;
+        t.sync();
+        int left = m;
+        // Round number r's key of contact c is (r << 21) | (2^21 - 1 - c) (contacts
+        // number below 2^21): the largest key a body receives in a round is its earliest
+        // pending contact, and keys of earlier rounds are smaller, so head[] needs
+        // clearing only when the round number wraps (every 2047 rounds).
+        unsigned round = 0;
+        for (int par = 0; left > 0; par ^= 1) {
+            if (++round == 2048u) {
+                for (int i = tid; i < n; i += T) hk[i] = 0u;
+                t.sync();
+                round = 1;
+            }
+            const unsigned rk = (round << 21) | 0x1FFFFFu;
+            auto claim = [&](int c, int s) {
+                atomicMax(&hk[s & 0xFFFF], rk - (unsigned)c);
+                if (s >= 0) atomicMax(&hk[s >> 16], rk - (unsigned)c);
+            };
+#pragma unroll
+            for (int r = 0; r < REG; ++r)
+                if ((pend >> r) & 1) claim(tid + r * T, slots[r]);
+            for (int c = tid + REG * T; c < m; c += T)
+                if (!done[c]) claim(c, pack(c));
+            t.sync();
+            auto ready = [&](int c, int s) {
+                const unsigned kc = rk - (unsigned)c;
+                if (hk[s & 0xFFFF] != kc || (s >= 0 && hk[s >> 16] != kc)) return false;
+                const int i = atomicAdd(&count[par], 1);
+                list[2 * i] = c;
+                list[2 * i + 1] = s;
+                return true;
+            };
+#pragma unroll
+            for (int r = 0; r < REG; ++r)
+                if (((pend >> r) & 1) && ready(tid + r * T, slots[r])) pend &= ~(1u << r);
+            for (int c = tid + REG * T; c < m; c += T)
+                if (!done[c] && ready(c, pack(c))) done[c] = 1;
+            if (tid == 0) count[par ^ 1] = 0;  // read last before this round's first sync
+            t.sync();
+            const int nr = count[par];
+            left -= nr;
+            for (int i = tid >> 2; i < nr; i += T >> 2) {
+                const int c = list[2 * i], s = list[2 * i + 1];
+                quad_apply<WARM>(B, s & 0xFFFF, s < 0 ? -1 : s >> 16, ts.quad(c), k, Cf, Cr,
+                                 WARM ? warm + 3 * (base + c) : nullptr, keep_dl ? &con(base + c).dln : nullptr);
+            }
+        }
+        t.sync();
+    }
+}
+
+// The same rounds with a contact per thread, for the plain step's large worlds, whose
+// rounds ready thousands of contacts and whose bodies and terms outgrow the LDS.
+// done[] for ncon.  con(c) is contact c's record (DirectCon).
+constexpr int SOLVE_TEAM_REG = 2;
+
+template <bool WARM, int REG, class Con>
 __device__ inline void solve_team(const Team &t, const Planes &B, int n, const Con &con, int ncon, int *done,
                                   int *head, const FloorDev &fl, const StepConsts &k, float Cf, float Cr,
-                                  const PreTerms &pre = PreTerms{}, float *warm = nullptr)
+                                  float *warm)
 {
     const int tid = t.rank, BLOCK = t.size;
-    const int npre = min(pre.na + pre.nb, ncon);
-    for (int c = tid; c < npre; c += BLOCK) contact_terms(B, con(c), fl, k, pre(c));
     // a thread's first REG contacts live in registers: their bodies, and
-    // the impulses they apply, written back once after the rounds (no global
-    // memory access on a round's critical path when their terms are in pre[])
+    // the impulses they apply, written back once after the rounds
     int sa[REG], sb[REG];
     bool pend[REG];
     float dl[REG][3];
@@ -240,10 +453,7 @@ __device__ inline void solve_team(const Team &t, const Planes &B, int n, const C
         dl[r][0] = dl[r][1] = dl[r][2] = 0.0f;
     }
     for (int c = tid + REG * BLOCK; c < ncon; c += BLOCK) done[c] = 0;
-    // Round k's key of contact c is (k << 21) | (2^21 - 1 - c) (contacts number
-    // below 2^21 on both paths): the largest key a body receives in round k is its
-    // earliest pending contact, and keys of earlier rounds are smaller, so head[]
-    // needs clearing only when the round number wraps (every 2047 rounds).
+    // keys as solve_packed's
     unsigned *hk = reinterpret_cast<unsigned *>(head);
     for (int i = tid; i < n; i += BLOCK) hk[i] = 0u;
     t.sync();
@@ -277,8 +487,7 @@ __device__ inline void solve_team(const Team &t, const Planes &B, int n, const C
         auto apply = [&](int c) {
             ContactRec r = con(c);
             float *sums = WARM ? warm + 3 * c : nullptr;
-            if (c < npre) contact_apply(B, r, pre(c), k, Cf, Cr, sums);
-            else constraint(B, r, fl, k, Cf, Cr, sums);
+            constraint(B, r, fl, k, Cf, Cr, sums);
             con(c).dln = r.dln;
             con(c).dlt1 = r.dlt1;
             con(c).dlt2 = r.dlt2;
@@ -289,16 +498,8 @@ __device__ inline void solve_team(const Team &t, const Planes &B, int n, const C
                 const int c = tid + r * BLOCK;
                 const unsigned kc = key(c);
                 if (hk[sa[r]] == kc && (sb[r] < 0 || hk[sb[r]] == kc)) {
-                    ContactRec rr;
-                    float *sums = WARM ? warm + 3 * c : nullptr;
-                    if (c < npre) {
-                        rr.slot_a = sa[r];
-                        rr.slot_b = sb[r];
-                        contact_apply(B, rr, pre(c), k, Cf, Cr, sums);
-                    } else {
-                        rr = con(c);
-                        constraint(B, rr, fl, k, Cf, Cr, sums);
-                    }
+                    ContactRec rr = con(c);
+                    constraint(B, rr, fl, k, Cf, Cr, WARM ? warm + 3 * c : nullptr);
                     dl[r][0] = rr.dln;
                     dl[r][1] = rr.dlt1;
                     dl[r][2] = rr.dlt2;
@@ -330,14 +531,6 @@ __device__ inline void solve_team(const Team &t, const Planes &B, int n, const C
             con(c).dlt2 = dl[r][2];
         }
     }
-}
-
-template <int BLOCK, bool WARM = false, class Con>
-__device__ inline void solve_rounds(const Planes &B, int n, const Con &con, int ncon, int *done, int *head,
-                                    const FloorDev &fl, const StepConsts &k, float Cf, float Cr,
-                                    const PreTerms &pre = PreTerms{}, float *warm = nullptr)
-{
-    solve_team<WARM>(Team::block(BLOCK), B, n, con, ncon, done, head, fl, k, Cf, Cr, pre, warm);
 }
 
 // ------------------------------------------------------------------ plain path kernels
@@ -491,7 +684,7 @@ struct SolveArgs {
     StepConsts k;
     const FloorDev *fl;
     float Cf, Cr;
-    int npre;             // contact terms kept in the dynamic LDS after head[]
+    int nterms;           // contact terms that the dynamic LDS has room for
     ContactRec *rec_out;  // recording (may be null)
     int rec_cap;
     int *rec_count;
@@ -511,10 +704,9 @@ struct SolveArgs {
 };
 
 // Ordered contact compaction, dependency-round solve and IntegrateVelocities of
-// one world, by one workgroup of T threads; head[] in dynamic LDS, followed by
-// npre contact terms (T = PLAIN_SMALL_THREADS for small worlds, whose 256 threads
-// have the registers to keep the terms' application free of spills; the
-// 1024-thread variant for large worlds keeps none).
+// one world, by one workgroup of T threads.  Worlds of at most PLAIN_SMALL_BODIES
+// bodies (T = PLAIN_SMALL_THREADS): bodies, lists and the terms of nterms contacts at a
+// time in dynamic LDS (solve_packed); larger ones: head[] there (solve_team).
 template <bool WARM, int T = SOLVE_THREADS>
 __global__ __launch_bounds__(T) void k_plain_solve(SolveArgs a)
 {
@@ -558,14 +750,20 @@ __global__ __launch_bounds__(T) void k_plain_solve(SolveArgs a)
         }
         __syncthreads();
     }
-    if constexpr (T == SOLVE_THREADS) {  // no terms kept: the path that applies them is not compiled
-        solve_rounds<T, WARM>(a.B, a.n, DirectCon{a.con}, ncon, a.done, head, fl, a.k, a.Cf, a.Cr, PreTerms{},
-                              a.warm_sums);
+    Planes Bv = a.B;
+    if constexpr (T == SOLVE_THREADS) {
+        solve_team<WARM, SOLVE_TEAM_REG>(Team::block(T), a.B, a.n, DirectCon{a.con}, ncon, a.done, head, fl, a.k, a.Cf,
+                                         a.Cr, a.warm_sums);
     } else {
-        PreTerms pre;
-        pre.a = reinterpret_cast<ContactTerms *>(head + ((a.n + 3) & ~3));
-        pre.na = a.npre;
-        solve_rounds<T, WARM>(a.B, a.n, DirectCon{a.con}, ncon, a.done, head, fl, a.k, a.Cf, a.Cr, pre, a.warm_sums);
+        const int rows = (a.n + 3) & ~3;
+        Bv = Planes{reinterpret_cast<float *>(head) + 3 * rows + 4, rows};
+        for (int i = threadIdx.x; i < a.n; i += T)
+#pragma unroll
+            for (int f = 0; f < F_NLDS; ++f) Bv.at(f, i) = a.B.at(f, i);
+        __syncthreads();
+        const LdsTerms ts{reinterpret_cast<ContactTerms *>(Bv.base + F_NLDS * rows), a.nterms};
+        solve_packed<WARM, SOLVE_REG>(Team::block(T), Bv, a.n, DirectCon{a.con}, ncon, a.done, head, head + rows + 4,
+                                      head + rows, ts, fl, a.k, a.Cf, a.Cr, a.warm_sums, a.rec_out != nullptr);
     }
     if (WARM) {
         __syncthreads();
@@ -577,8 +775,12 @@ __global__ __launch_bounds__(T) void k_plain_solve(SolveArgs a)
         if (threadIdx.x == 0) *a.warm_n_next = m;
     }
     for (int i = threadIdx.x; i < a.n; i += T) {
-        if (a.k.quat) integrate_velocities_quat(a.B, a.B, i, a.k.dt);
-        else integrate_velocities_body(a.B, i, a.k.dt);
+        if (a.k.quat) integrate_velocities_quat(Bv, a.B, i, a.k.dt);
+        else integrate_velocities_body(Bv, i, a.k.dt);
+        if constexpr (T != SOLVE_THREADS) {
+#pragma unroll
+            for (int f = 0; f < F_SX; ++f) a.B.at(f, i) = Bv.at(f, i);
+        }
     }
     if (a.rec_out) {
         __syncthreads();
@@ -851,14 +1053,21 @@ __device__ __forceinline__ void batched_world(const BatchArgsT<WARM> &a, const T
     }
     const float Cf = a.wfric ? a.wfric[w] : a.k.friction;
     const float Cr = a.wrest ? a.wrest[w] : a.k.restitution;
-    // contact terms in the radii, then in the team's polytope LDS
-    PreTerms pre;
-    pre.a = reinterpret_cast<ContactTerms *>(L.brad);
-    pre.na = (int)(sizeof(float) * L.rows / sizeof(ContactTerms));
-    pre.b = reinterpret_cast<ContactTerms *>(epa);
-    pre.nb = (int)(NW * sizeof(EpaLds) / sizeof(ContactTerms));
-    solve_team<WARM, BATCH_SOLVE_REG>(t, Lb, n, DirectCon{con}, ncon, done, L.head, fl, a.k, Cf, Cr, pre,
-                                      WARM ? wsum : nullptr);
+    // the solver's lists in the team's polytope LDS, contact terms in the radii, in the
+    // rest of the polytope LDS, then in rec[]'s memory after the accumulators
+    int *list = reinterpret_cast<int *>(epa);
+    const int lw = (2 * n + 2 + 3) & ~3;
+    constexpr int TW = (int)(sizeof(ContactTerms) / sizeof(float));
+    float *gt = reinterpret_cast<float *>(rec) + (WARM ? 3 * ncon : 0);
+    SplitTerms ts;
+    ts.a = reinterpret_cast<ContactTerms *>(L.brad);
+    ts.na = L.rows / TW;
+    ts.b = reinterpret_cast<ContactTerms *>(list + lw);
+    ts.nb = (NW * (int)(sizeof(EpaLds) / sizeof(float)) - lw) / TW;
+    ts.g = reinterpret_cast<ContactTerms *>(gt);
+    ts.ng = (S.cap * (int)(sizeof(ContactRec) / sizeof(float)) - (WARM ? 3 * ncon : 0)) / TW;
+    solve_packed<WARM, SOLVE_REG>(t, Lb, n, DirectCon{con}, ncon, done, L.head, list + 2, list, ts, fl, a.k, Cf, Cr,
+                                  WARM ? wsum : nullptr, a.rec_out != nullptr);
     if constexpr (WARM) {  // this step's list: the first warm_cap[w] contacts (contact c's sums are team thread c % T's)
         const int64_t off = a.warm_off[w];
         const bool odd = (a.warm_flip + step) & 1;
@@ -1478,7 +1687,7 @@ int nans_upload_worlds(nans_ctx *ctx, int32_t nworlds, const int32_t *world_offs
     for (const void *f : {(const void *)k_plain_solve<false, PLAIN_SMALL_THREADS>,
                           (const void *)k_plain_solve<true, PLAIN_SMALL_THREADS>})
         NANS_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                     (int)(sizeof(int) * PLAIN_SMALL_BODIES + sizeof(ContactTerms) * PLAIN_SMALL_TERMS)));
+                                     (int)PLAIN_SMALL_LDS));
     k_zero_u64<<<1, 64>>>(W->cnt, CNT_N);
     NANS_HIP(hipGetLastError());
     NANS_TRY(setup_floor(ctx, nullptr));
@@ -1697,10 +1906,15 @@ int nans_step_plain(nans_ctx *ctx, int32_t nsteps)
             a.rec_count = W->record ? W->rec_count + w : nullptr;
             a.cnt = W->cnt;
             a.cand = cand;
-            // worlds of at most PLAIN_SMALL_BODIES bodies: 256 threads, contact terms in LDS
+            // worlds of at most PLAIN_SMALL_BODIES bodies: 256 threads, bodies and contact terms in LDS
             const bool small = n <= PLAIN_SMALL_BODIES;
-            a.npre = small ? PLAIN_SMALL_TERMS : 0;
-            const size_t lds = sizeof(int) * (size_t)((n + 3) & ~3) + sizeof(ContactTerms) * (size_t)a.npre;
+            const int rows = (n + 3) & ~3;
+            const size_t head_bytes = sizeof(int) * (size_t)rows;
+            const size_t fixed = plain_small_fixed_bytes(n);
+            a.nterms = small ? (int)std::max<int64_t>(
+                                   1, std::min<int64_t>((PLAIN_SMALL_LDS - fixed) / sizeof(ContactTerms), npairs))
+                             : 0;
+            const size_t lds = small ? fixed + sizeof(ContactTerms) * (size_t)a.nterms : head_bytes;
             if (ctx->warm) {
                 const int cur = W->warm_flip, nxt = cur ^ 1;
                 const int64_t off = W->h_warm_off[w];
