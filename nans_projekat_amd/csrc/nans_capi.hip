@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PE
         if (base >= n) break;
         const int count = (int)min((int64_t)share, n - base);
         PairSrc src{a, b, base, n, o, &cnt[0], sim + base};
-        narrow_wave<true, ISL>(src, count, p, lds[wv], list + base, found);
+        narrow_wave<ISL>(src, count, p, lds[wv], list + base, found);
     }
 }
 

@@ -81,7 +81,7 @@ struct Team {
     __device__ static Team block(int threads) { return Team{(int)threadIdx.x, threads, true}; }
     __device__ static Team wave() { return Team{(int)(threadIdx.x & 63), 64, false}; }
     __device__ int waves() const { return size >> 6; }
-    __device__ void sync() const
+    __device__ __forceinline__ void sync() const
     {
         if (whole) {
             __syncthreads();
@@ -92,7 +92,7 @@ struct Team {
         }
     }
     // sync() that also returns the number of threads with p set
-    __device__ int sync_count(bool p) const
+    __device__ __forceinline__ int sync_count(bool p) const
     {
         if (whole) return __syncthreads_count(p);
         const int c = __popcll(__ballot(p));
@@ -171,7 +171,7 @@ struct EpaShapes {
     V3 k;                // lanes 0-7: corner (lane) of A; lanes 8-15: corner (lane - 8) of B
 };
 
-__device__ inline V3 pick_corner(const Shape &s, int k)
+__device__ __forceinline__ V3 pick_corner(const Shape &s, int k)
 {
     V3 v = s.v[0];
 #pragma unroll
@@ -184,7 +184,7 @@ __device__ inline V3 pick_corner(const Shape &s, int k)
     return v;
 }
 
-__device__ inline EpaShapes epa_shapes(const Shape &A, const Shape &B)
+__device__ __forceinline__ EpaShapes epa_shapes(const Shape &A, const Shape &B)
 {
     const int lane = lane_id();
     EpaShapes e;
@@ -204,9 +204,8 @@ __device__ inline EpaShapes epa_shapes(const Shape &A, const Shape &B)
 // along -d), both at once: in each group of 8 lanes, the first corner of greatest
 // dot(v, dir) among those above -FLT_MAX, else (0,0,0) -- GetCubeSupport's strict
 // '>' scan from -FLT_MAX (code/nans.cpp:409-430).
-__device__ __forceinline__ void box_supports(V3 kv, V3 d, V3 nd, V3 &sa, V3 &sb)
+__device__ __forceinline__ void box_supports(V3 kv, V3 d, V3 nd, V3 &sa, V3 &sb, int lane)
 {
-    const int lane = lane_id();
     const float dist = dot(kv, lane >= 8 ? nd : d);
     float key = dist > -FLT_MAX ? dist : -__builtin_inff();
     int idx = lane & 7;
@@ -227,12 +226,12 @@ __device__ __forceinline__ void box_supports(V3 kv, V3 d, V3 nd, V3 &sa, V3 &sb)
 }
 
 // CalculateSupport (code/nans.cpp:463-519): S_A(d) and S_B(-d); every lane calls.
-__device__ inline Vtx wave_support(const EpaShapes &s, V3 d)
+__device__ __forceinline__ Vtx wave_support(const EpaShapes &s, V3 d, int lane)
 {
     const V3 nd = mul(d, -1.0f);
     Vtx v;
     V3 ga = mk3(0.0f, 0.0f, 0.0f), gb = mk3(0.0f, 0.0f, 0.0f);
-    if (s.kind_a == SHAPE_BOX || s.kind_b == SHAPE_BOX) box_supports(s.k, d, nd, ga, gb);
+    if (s.kind_a == SHAPE_BOX || s.kind_b == SHAPE_BOX) box_supports(s.k, d, nd, ga, gb, lane);
     v.A = s.kind_a == SHAPE_BOX ? ga : sphere_support(s.ca, s.ra, d);
     v.B = s.kind_b == SHAPE_BOX ? gb : sphere_support(s.cb, s.rb, nd);
     v.P = sub(v.A, v.B);
@@ -261,10 +260,9 @@ __device__ __forceinline__ int nth_set_bit(uint64_t m, int n)
 // Equality class of a new vertex with id nv and point P against the vertices in
 // registers (vertex == compares P, code/nans.h:251-254): the first earlier vertex
 // with the same P, CLS_NAN if P has a NaN.  Every lane calls.
-__device__ __forceinline__ int vertex_class_reg(V3 v0, V3 v1, int nv, V3 P)
+__device__ __forceinline__ int vertex_class_reg(V3 v0, V3 v1, int nv, V3 P, int lane)
 {
     if (has_nan(P)) return CLS_NAN;
-    const int lane = lane_id();
     const uint64_t m0 = ballot(lane < nv && veq(v0, P));
     if (m0) return ffs64(m0);
     const uint64_t m1 = ballot(lane + 64 < nv && veq(v1, P));
@@ -297,26 +295,30 @@ __device__ __forceinline__ FaceR make_face(V3 A, V3 B, V3 C, int a, int b, int c
     return f;
 }
 
-// Binary64 distance of a face's plane to the origin (FP64-islands final choice).
+// Binary64 distance of the plane of A, B, C to the origin (FP64-islands final choice).
+__device__ inline double face_plane64(V3 A, V3 B, V3 C)
+{
+    const double ax = A.x, ay = A.y, az = A.z;
+    const double ux = (double)B.x - ax, uy = (double)B.y - ay, uz = (double)B.z - az;
+    const double vx = (double)C.x - ax, vy = (double)C.y - ay, vz = (double)C.z - az;
+    const double nx = uy * vz - vy * uz, ny = uz * vx - vz * ux, nz = ux * vy - vx * uy;
+    const double inv = 1.0 / __builtin_sqrt((nx * nx + ny * ny) + nz * nz);
+    const double d = ((nx * inv) * ax + (ny * inv) * ay) + (nz * inv) * az;
+    return d >= 0.0 ? d : -d;
+}
+
+// The same for a face of the whole-wave polytope.
 __device__ inline double face_dist64(const EpaLds &L, const FaceR &f)
 {
-    int b = (f.id >> 8) & 255, c = (f.id >> 16) & 255;
-    double ax = f.ax, ay = f.ay, az = f.az;
-    double ux = (double)L.vp[b][0] - ax, uy = (double)L.vp[b][1] - ay, uz = (double)L.vp[b][2] - az;
-    double vx = (double)L.vp[c][0] - ax, vy = (double)L.vp[c][1] - ay, vz = (double)L.vp[c][2] - az;
-    double nx = uy * vz - vy * uz, ny = uz * vx - vz * ux, nz = ux * vy - vx * uy;
-    double inv = 1.0 / __builtin_sqrt((nx * nx + ny * ny) + nz * nz);
-    double d = ((nx * inv) * ax + (ny * inv) * ay) + (nz * inv) * az;
-    return d >= 0.0 ? d : -d;
+    return face_plane64(mk3(f.ax, f.ay, f.az), ld3(L.vp, (f.id >> 8) & 255), ld3(L.vp, (f.id >> 16) & 255));
 }
 
 // ResolveCollision (code/nans.cpp:787-904) executed by one full wavefront.  The
 // caller has written the GJK simplex to L.vp / L.va / L.vb[0..3], passes vertex
 // (lane)'s P in p0 for lanes 0-3, and has called wave_sync().  Every lane returns
 // the same result.
-__device__ __forceinline__ EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, const NarrowParams &p)
+__device__ __forceinline__ EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3 p0, const NarrowParams &p, int lane)
 {
-    const int lane = lane_id();
     EpaResult r;
     r.status = EPA_ITER;
     r.pa = r.pb = r.n = mk3(0.0f, 0.0f, 0.0f);
@@ -387,7 +389,7 @@ __device__ __forceinline__ EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3
                    readlane_f(pick3f(ks, F[0].nz, F[1].nz, F[2].nz), owner));
         float cur = m == __builtin_inff() ? d0 : readlane_f(pick3f(ks, F[0].d, F[1].d, F[2].d), owner);
         // new support along the stored normal
-        const Vtx ns = wave_support(sh, N);
+        const Vtx ns = wave_support(sh, N, lane);
         if (dot(N, ns.P) - cur < p.epa_tolerance) {
             double depth = (double)cur;
             if (p.fp64_islands) {
@@ -453,7 +455,7 @@ __device__ __forceinline__ EpaResult epa_wave(EpaLds &L, const EpaShapes &sh, V3
         }
         // append the vertex
         const int vnew = nv;
-        const int ncls = vertex_class_reg(v0, v1, vnew, ns.P);
+        const int ncls = vertex_class_reg(v0, v1, vnew, ns.P, lane);
         if (lane == (vnew & 63)) {
             if (vnew < 64) v0 = ns.P;
             else v1 = ns.P;
@@ -740,9 +742,9 @@ __device__ __forceinline__ V3 gbcast3(V3 v)
 
 // this lane's G-lane group bits of a wave ballot
 template <int G>
-__device__ __forceinline__ uint32_t gbits(uint64_t m)
+__device__ __forceinline__ uint32_t gbits(uint64_t m, int lane)
 {
-    return (uint32_t)(m >> (lane_id() & (64 - G))) & (uint32_t)((1ull << G) - 1ull);
+    return (uint32_t)(m >> (lane & (64 - G))) & (uint32_t)((1ull << G) - 1ull);
 }
 // minimum over the lane's group of G (no NaN inputs), in every lane of the group:
 // a row of 16 by DPP, then the two rows of a 32-lane group through ds_bpermute
@@ -761,9 +763,9 @@ __device__ __forceinline__ float group_min(float v)
 // MEM: the shapes carry only Shape::vm (corners in memory, null for a sphere),
 // and each lane reads its one corner from there.
 template <bool MEM = false>
-__device__ inline EpaShapes epa_shapes_group(const Shape &A, const Shape &B)
+__device__ __forceinline__ EpaShapes epa_shapes_group(const Shape &A, const Shape &B, int lane = lane_id())
 {
-    const int j = lane_id() & 15;
+    const int j = lane & 15;
     EpaShapes e;
     e.kind_a = A.kind;
     e.kind_b = B.kind;
@@ -789,9 +791,9 @@ __device__ inline EpaShapes epa_shapes_group(const Shape &A, const Shape &B)
 // order -- and a row mirror hands each half the other half's winner.  No
 // cross-lane traffic leaves the row, so a 32-lane group's two rows agree.
 template <int G>
-__device__ inline Vtx group_support(const EpaShapes &s, V3 d)
+__device__ __forceinline__ Vtx group_support(const EpaShapes &s, V3 d, int lane)
 {
-    const int lane = lane_id(), j = lane & 15;
+    const int j = lane & 15;
     const V3 nd = mul(d, -1.0f);
     const float dist = dot(s.k, j >= 8 ? nd : d);
     float key = dist > -FLT_MAX ? dist : -__builtin_inff();
@@ -840,20 +842,13 @@ __device__ __forceinline__ int edge_key(int cl, int e)
 // choice), its vertices b and c from the group's vertex LDS.
 __device__ inline double group_face_dist64(const float (*vp)[3], const FaceR &f)
 {
-    const int b = (f.id >> 8) & 255, c = (f.id >> 16) & 255;
-    const double ax = f.ax, ay = f.ay, az = f.az;
-    const double ux = (double)vp[b][0] - ax, uy = (double)vp[b][1] - ay, uz = (double)vp[b][2] - az;
-    const double vx = (double)vp[c][0] - ax, vy = (double)vp[c][1] - ay, vz = (double)vp[c][2] - az;
-    const double nx = uy * vz - vy * uz, ny = uz * vx - vz * ux, nz = ux * vy - vx * uy;
-    const double inv = 1.0 / __builtin_sqrt((nx * nx + ny * ny) + nz * nz);
-    const double d = ((nx * inv) * ax + (ny * inv) * ay) + (nz * inv) * az;
-    return d >= 0.0 ? d : -d;
+    return face_plane64(mk3(f.ax, f.ay, f.az), ld3(vp, (f.id >> 8) & 255), ld3(vp, (f.id >> 16) & 255));
 }
 
 // Argmin over (value, index) in each G-lane group, ties to the lowest index;
 // every lane of the group receives the result.
 template <int G>
-__device__ inline void group_argmin64(bool &valid, double &v, int &i)
+__device__ __forceinline__ void group_argmin64(bool &valid, double &v, int &i)
 {
 #pragma unroll
     for (int off = 1; off < G; off <<= 1) {
@@ -871,10 +866,10 @@ __device__ inline void group_argmin64(bool &valid, double &v, int &i)
 // (as epa_wave's).
 template <int G, bool ISL = false>
 __device__ __forceinline__ EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh, V3 sa0, V3 sb0, bool act,
-                                      const NarrowParams &p)
+                                      const NarrowParams &p, int lane)
 {
-    const int lane = lane_id(), j = lane & (G - 1), gb = lane & (64 - G), g = lane / G;
-    auto gbits = [](uint64_t m) { return nans::gbits<G>(m); };
+    const int j = lane & (G - 1), gb = lane & (64 - G), g = lane / G;
+    auto gbits = [lane](uint64_t m) { return nans::gbits<G>(m, lane); };
     EpaResult r;
     r.status = act ? EPA_ITER : EPA_NONE;
     r.pa = r.pb = r.n = mk3(0.0f, 0.0f, 0.0f);
@@ -974,7 +969,7 @@ __device__ __forceinline__ EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh
         const V3 N = mk3(gpull_f(F.nx, owner), gpull_f(F.ny, owner), gpull_f(F.nz, owner));
         const float cur = m == __builtin_inff() ? d0 : m;
         // new support along the stored normal
-        const Vtx ns = group_support<G>(sh, N);
+        const Vtx ns = group_support<G>(sh, N, lane);
         const bool conv = run && dot(N, ns.P) - cur < p.epa_tolerance;
         if (ballot(conv)) {
             const int fid = gpull_i(F.id, owner);
@@ -1138,6 +1133,289 @@ __device__ __forceinline__ EpaResult epa_group(EpgLds<G> &L, const EpaShapes &sh
     return r;
 }
 
+// ---------------------------------------------------------------------- an EPA per lane
+// ResolveCollision for one pair of boxes by one lane: the step's contacts are shallow
+// and end after a few iterations (of a batch of stacks' GJK hits 34 % after one, 95 %
+// after four, 99.3 % after five), so a polytope of at most 8 vertices and 12 faces is
+// small enough to keep EPL_LANES of them in a wave's polytope LDS, one lane's words
+// EPL_LANES apart.  A trip then costs a wave about 1.3k instructions for up to
+// EPL_LANES pairs, where the 16-lane groups spend 1k on four (their lanes past the
+// polytope's faces idle, and every gather crosses lanes): 4096 worlds of 8-256 bodies
+// 81.0 -> 67.8 ms per 60 steps, 601 with warm start 31.5 -> 25.6 ms per 30.  What outgrows a lane -- a
+// ninth vertex, a thirteenth face, a ninth horizon edge, a NaN vertex -- goes to the
+// wider tiers, as pairs with a sphere do.
+constexpr int EPL_V = 8, EPL_F = 12;
+constexpr int EPL_WORDS = 3 * EPL_V + 5 * EPL_F;  // vertices P, then faces: N, distance, vertex ids
+constexpr int EPL_LANES = 24;
+static_assert(4 * EPL_WORDS * EPL_LANES <= sizeof(EpaLds), "the lane polytopes fit the wave's EPA LDS");
+
+struct EpaLane {
+    float *w;            // the lane's words in LDS
+    const float *va, *vb;  // the boxes' corners in memory
+    int nf, nv, iter;
+    unsigned long long ord;  // slot of the face at position i of the vector in bits 4i
+    unsigned used;       // the slots that hold a face
+    unsigned cls;        // equality class of vertex v in bits 4v
+    unsigned sup;        // corners (8: none) of vertex 4 + k: A's in bits 8k, B's in 8k + 4
+    int best;            // the closest face's slot, once the pair has converged
+
+    __device__ float &at(int i) const { return w[i * EPL_LANES]; }
+    __device__ V3 p(int v) const { return mk3(at(3 * v), at(3 * v + 1), at(3 * v + 2)); }
+    __device__ void put(int v, V3 q) const
+    {
+        at(3 * v) = q.x;
+        at(3 * v + 1) = q.y;
+        at(3 * v + 2) = q.z;
+    }
+    static __device__ int face(int f) { return 3 * EPL_V + 5 * f; }
+    __device__ V3 normal(int f) const { return mk3(at(face(f)), at(face(f) + 1), at(face(f) + 2)); }
+    __device__ float dist(int f) const { return at(face(f) + 3); }
+    __device__ int ids(int f) const { return __float_as_int(at(face(f) + 4)); }
+    // PushTriangle (code/nans.cpp:291-322) in slot f
+    __device__ __forceinline__ void push(int f, V3 A, V3 B, V3 C, int a, int b, int c) const
+    {
+        float d;
+        const V3 n = plane(A, B, C, d);
+        store(f, n, d, a | (b << 4) | (c << 8));
+    }
+    static __device__ __forceinline__ V3 plane(V3 A, V3 B, V3 C, float &dist)
+    {
+        V3 n = normalize(cross(sub(B, A), sub(C, A)));
+        const float d = dot(n, A);
+        if (d < 0.0f) n = mul(n, -1.0f);
+        dist = gabs(d);
+        return n;
+    }
+    __device__ __forceinline__ void store(int f, V3 n, float d, int ids) const
+    {
+        const int o = face(f);
+        at(o) = n.x;
+        at(o + 1) = n.y;
+        at(o + 2) = n.z;
+        at(o + 3) = d;
+        at(o + 4) = __int_as_float(ids);
+    }
+};
+
+// The corner of a box in memory that box_support picks, 8 for none.
+__device__ __forceinline__ int corner_support(const float *v, V3 d, V3 &best)
+{
+    float maxd = -FLT_MAX;
+    int idx = 8;
+    best = mk3(0.0f, 0.0f, 0.0f);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const V3 c = mk3(v[3 * k], v[3 * k + 1], v[3 * k + 2]);
+        const float dist = dot(c, d);
+        const bool t = dist > maxd;
+        maxd = t ? dist : maxd;
+        idx = t ? k : idx;
+        fsel(best, t, c);
+    }
+    return idx;
+}
+
+// The simplex of a queued hit as the lane's polytope; false if it has a NaN.
+__device__ __forceinline__ bool epa_lane_start(EpaLane &e, const float *qa, const float *qb)
+{
+    V3 P[4];
+    bool ok = true;
+    e.cls = 0;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        P[v] = sub(mk3(qa[3 * v], qa[3 * v + 1], qa[3 * v + 2]), mk3(qb[3 * v], qb[3 * v + 1], qb[3 * v + 2]));
+        ok = ok && !has_nan(P[v]);
+        int c = v;
+#pragma unroll
+        for (int u = v - 1; u >= 0; --u) c = veq(P[u], P[v]) ? u : c;
+        e.cls |= (unsigned)c << (4 * v);
+        e.put(v, P[v]);
+    }
+    // ABC, ACD, ADB, BDC (code/nans.cpp:799-802)
+    e.push(0, P[0], P[1], P[2], 0, 1, 2);
+    e.push(1, P[0], P[2], P[3], 0, 2, 3);
+    e.push(2, P[0], P[3], P[1], 0, 3, 1);
+    e.push(3, P[1], P[3], P[2], 1, 3, 2);
+    e.nf = e.nv = 4;
+    e.ord = 0x3210;
+    e.used = 0xF;
+    e.iter = 0;
+    e.sup = 0;
+    return ok;
+}
+
+// One iteration of the loop (code/nans.cpp:804-902): EPA_NONE to go on, EPA_CONTACT
+// once converged (e.best then is the closest face), another status if the loop ended,
+// or EPA_SPILL.
+__device__ __forceinline__ int epa_lane_trip(EpaLane &e, const NarrowParams &np)
+{
+    if (!(e.iter <= np.max_epa_iterations)) return EPA_ITER;
+    e.iter += 1;
+    if (e.nf == 0) return EPA_EMPTY;
+    // closest face: the strict '<' scan from the first one
+    int best = (int)e.ord & 15;
+    float cur = e.dist(best);
+    for (int i = 1; i < e.nf; i += 4) {
+        const unsigned o = (unsigned)(e.ord >> (4 * i));
+        float d[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d[k] = e.dist((int)(o >> (4 * k)) & 15);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const bool t = i + k < e.nf && d[k] < cur;
+            best = t ? (int)(o >> (4 * k)) & 15 : best;
+            cur = t ? d[k] : cur;
+        }
+    }
+    const V3 N = e.normal(best);
+    V3 A, B;
+    const int ia = corner_support(e.va, N, A);
+    const int ib = corner_support(e.vb, mul(N, -1.0f), B);
+    const V3 P = sub(A, B);
+    if (dot(N, P) - cur < np.epa_tolerance) {
+        e.best = best;
+        return EPA_CONTACT;
+    }
+    if (e.nv >= EPL_V || has_nan(P)) return EPA_SPILL;
+    // append the vertex
+    const int vnew = e.nv;
+    int nc = vnew;
+#pragma unroll
+    for (int v = EPL_V - 2; v >= 0; --v) nc = v < vnew && veq(e.p(v), P) ? v : nc;
+    e.cls |= (unsigned)nc << (4 * vnew);
+    e.sup |= (unsigned)(ia | (ib << 4)) << (8 * (vnew - 4));
+    e.put(vnew, P);
+    e.nv = vnew + 1;
+    // visible faces, a bit per position
+    unsigned vis = 0;
+    for (int i = 0; i < e.nf; i += 2) {
+        const unsigned o = (unsigned)(e.ord >> (4 * i));
+        V3 n[2], a[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int f = (int)(o >> (4 * k)) & 15;
+            n[k] = e.normal(f);
+            a[k] = e.p(e.ids(f) & 7);
+        }
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            vis |= (i + k < e.nf && dot(n[k], sub(P, a[k])) > 0.0f) ? 1u << (i + k) : 0u;
+    }
+    // their directed edges as a set, bit 8 ca + cb; an edge pushed twice spills
+    unsigned long long set = 0;
+    bool dup = false;
+    auto cls_of = [&](int v) { return (int)(e.cls >> (4 * v)) & 7; };
+    for (unsigned m = vis; m; m &= m - 1) {
+        const int id = e.ids((int)(e.ord >> (4 * __builtin_ctz(m))) & 15);
+        const int ca = cls_of(id & 15), cb = cls_of((id >> 4) & 15), cc = cls_of(id >> 8);
+        const unsigned long long b = (1ull << (8 * ca + cb)) | (1ull << (8 * cb + cc)) | (1ull << (8 * cc + ca));
+        dup |= (set & b) != 0;
+        set |= b;
+    }
+    // horizon (PushEdge, code/nans.cpp:232-266): in face order the edges whose reverse is
+    // not in the set; vertices of edge k in byte k
+    unsigned long long eids = 0;
+    int ne = 0;
+    for (unsigned m = vis; m; m &= m - 1) {
+        const int id = e.ids((int)(e.ord >> (4 * __builtin_ctz(m))) & 15);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int a = (id >> (4 * k)) & 15, b = (id >> (4 * ((k + 1) % 3))) & 15;
+            if (!((set >> (8 * cls_of(b) + cls_of(a))) & 1)) {
+                eids |= (unsigned long long)(unsigned)(a | (b << 4)) << ((8 * ne) & 63);
+                ne += 1;
+            }
+        }
+    }
+    if (dup || ne > 8 || e.nf - __popc(vis) + ne > EPL_F) return EPA_SPILL;
+    // the visible faces leave the vector, the new ones follow in edge order
+    int nf = e.nf;
+    for (unsigned m = vis; m;) {
+        const int i = 31 - __builtin_clz(m);
+        m ^= 1u << i;
+        e.used &= ~(1u << ((int)(e.ord >> (4 * i)) & 15));
+        const unsigned long long low = (1ull << (4 * i)) - 1ull;
+        e.ord = (e.ord & low) | ((e.ord >> 4) & ~low);
+        nf -= 1;
+    }
+    e.ord &= (1ull << (4 * nf)) - 1ull;
+    // two at a time, their chains side by side
+    for (int k = 0; k < ne; k += 2) {
+        const int ab = (int)(eids >> (8 * k)), a = ab & 7, b = (ab >> 4) & 7, a2 = (ab >> 8) & 7, b2 = (ab >> 12) & 7;
+        const V3 A0 = e.p(a), B0 = e.p(b), A1 = e.p(a2), B1 = e.p(b2);
+        float d0, d1;
+        const V3 n0 = EpaLane::plane(P, A0, B0, d0), n1 = EpaLane::plane(P, A1, B1, d1);
+        int f = __builtin_ctz(~e.used);
+        e.store(f, n0, d0, vnew | (a << 4) | (b << 8));
+        e.used |= 1u << f;
+        e.ord |= (unsigned long long)f << (4 * (nf + k));
+        if (k + 1 < ne) {
+            f = __builtin_ctz(~e.used);
+            e.store(f, n1, d1, vnew | (a2 << 4) | (b2 << 8));
+            e.used |= 1u << f;
+            e.ord |= (unsigned long long)f << (4 * (nf + k + 1));
+        }
+    }
+    e.nf = nf + ne;
+    return EPA_NONE;
+}
+
+// The contact of a converged lane (code/nans.cpp:826-866; ISL: the final face by
+// binary64 plane distance, as epa_group's).  qa, qb: the queued simplex's supports.
+template <bool ISL>
+__device__ __forceinline__ EpaResult epa_lane_finish(const EpaLane &e, const float *qa, const float *qb)
+{
+    EpaResult r;
+    r.pa = r.pb = r.n = mk3(0.0f, 0.0f, 0.0f);
+    int best = e.best;
+    r.depth = (double)e.dist(best);
+    if constexpr (ISL) {
+        double d0 = 0.0, bd = 0.0;
+        for (int i = 0; i < e.nf; ++i) {
+            const int f = (int)(e.ord >> (4 * i)) & 15, id = e.ids(f);
+            const double d = face_plane64(e.p(id & 15), e.p((id >> 4) & 15), e.p((id >> 8) & 15));
+            if (i == 0) d0 = bd = d;
+            if (i == 0 || (d < d0 && d < bd)) {
+                bd = d;
+                best = f;
+            }
+        }
+        r.depth = bd;
+    }
+    const V3 N = e.normal(best);
+    const int id = e.ids(best), a = id & 15, b = (id >> 4) & 15, c = (id >> 8) & 15;
+    const V3 PA = e.p(a), PB = e.p(b), PC = e.p(c);
+    // Barycentric (code/nans.cpp:771-785) of N * d
+    const V3 P = mul(N, e.dist(best));
+    const V3 e0 = sub(PB, PA), e1 = sub(PC, PA), e2 = sub(P, PA);
+    const float d00 = dot(e0, e0), d01 = dot(e0, e1), d11 = dot(e1, e1);
+    const float d20 = dot(e2, e0), d21 = dot(e2, e1);
+    const float denom = d00 * d11 - d01 * d01;
+    const float V = (d11 * d20 - d01 * d21) / denom;
+    const float W = (d00 * d21 - d01 * d20) / denom;
+    const float U = 1.0f - V - W;
+    if (fabsf(U) > 1.0f || fabsf(V) > 1.0f || fabsf(W) > 1.0f) {
+        r.status = EPA_BARY;
+    } else if (!isfinite(U) || !isfinite(V) || !isfinite(W)) {
+        r.status = EPA_NONFINITE;
+    } else {
+        // a vertex's supports: the simplex's from its record, the others' from the boxes
+        auto support = [&](const float *q, const float *box, int v, int shift) {
+            const int k = (int)(e.sup >> (8 * (v & 3) + shift)) & 15;
+            if (v >= 4 && k == 8) return mk3(0.0f, 0.0f, 0.0f);
+            const float *x = v < 4 ? q + 3 * v : box + 3 * k;
+            return mk3(x[0], x[1], x[2]);
+        };
+        r.pa = add(add(mul(support(qa, e.va, a, 0), U), mul(support(qa, e.va, b, 0), V)),
+                   mul(support(qa, e.va, c, 0), W));
+        r.n = mul(N, -1.0f);
+        r.pb = add(add(mul(support(qb, e.vb, a, 4), U), mul(support(qb, e.vb, b, 4), V)),
+                   mul(support(qb, e.vb, c, 4), W));
+        r.status = EPA_CONTACT;
+    }
+    return r;
+}
+
 // ---------------------------------------------------------------------- block driver
 // CheckCollision (code/nans.cpp:906-966) over the candidates [0, ncand) of one
 // workgroup, in two phases:
@@ -1176,12 +1454,23 @@ constexpr int GJK_CYCLE_START = 8;
 // the MI355X: 1.429 ms per step at 16, 1.413 at 32-56, 1.484 at 64).
 constexpr int GJK_REFILL_MIN = 48;
 
+// Candidates per wave up to which a team's EPA runs in 16-lane groups: the few hits of
+// so small a world leave most lanes idle, and a trip of the lanes' EPA lasts longer
+// (1024 worlds of 16 bodies, 29 candidates a wave, rollout and gradient: 24.4 ms with
+// lanes, 22.7 with groups; 48 worlds of 8-64, up to some 300 a wave: 4.9 against 6.7).
+constexpr int EPL_MIN = 48;
+
+// Lanes that wait for new pairs in the EPA phase before they are served, so that the
+// code that starts and ends pairs runs for several.
+constexpr int EPL_REFILL = 8;
+
 // A queued GJK hit's simplex: the supports on A and B of its four vertices (the
 // Minkowski point is recomputed as SupA - SupB, the expression that made it),
 // and the pair's key (the source's key(c)), so that EPA looks nothing else up.
 struct SimplexRec {
     float a[12], b[12];
     int key;
+    int next;  // chain of the slots whose pairs outgrew a lane (narrow_team)
 };
 
 __device__ __forceinline__ void simplex_rec_put(SimplexRec &q, const Vtx &v, int k)
@@ -1270,6 +1559,70 @@ __device__ __forceinline__ int gjk_lane_call(GjkLane &G, float *cyc, const Narro
     return GJK_STILL;
 }
 
+// EPA of one queued pair by the whole wave: supports of its four simplex vertices
+// in q, every lane returns the result.
+__device__ __forceinline__ EpaResult epa_whole(EpaLds &L, const EpaShapes &es, const SimplexRec &q, const NarrowParams &np,
+                                              int lane = lane_id())
+{
+    V3 p0 = mk3(0.0f, 0.0f, 0.0f);
+    if (lane < 4) {
+        const V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
+        const V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
+        p0 = sub(a, b);
+        st3(L.va, lane, a);
+        st3(L.vb, lane, b);
+        st3(L.vp, lane, p0);
+    }
+    wave_sync();
+    const EpaResult r = epa_wave(L, es, p0, np, lane);
+    wave_sync();
+    return r;
+}
+
+// Four queue slots (job, uniform over each 16-lane group; groups without act idle along
+// on a valid one) of candidates c in the 16-lane groups; one that outgrows its group by
+// the whole wave.  Between its shapes' set-up and its loop it calls next().
+template <bool ISL, class Src, class Next>
+__device__ __forceinline__ void epa_four(const Src &src, EpaLds &L, const SimplexRec *qsim, int job, int c, bool act,
+                                         const NarrowParams &np, int lane, Next &&next)
+{
+    const int j = lane & 15;
+    const SimplexRec &q = qsim[job];
+    const int key = q.key;
+    Shape A, B;
+    src.shapes_ref(key, A, B);
+    const EpaShapes es = epa_shapes_group<true>(A, B, lane);
+    V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
+    if (j < 4) {
+        sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
+        sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
+    }
+    wave_sync();
+    next();
+    const EpaResult r = epa_group<16, ISL>(*reinterpret_cast<EpgLds<16> *>(&L), es, sa0, sb0, act, np, lane);
+    if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
+    wave_sync();
+    for (uint64_t sp = ballot(act && j == 0 && r.status == EPA_SPILL); sp; sp &= sp - 1) {
+        const int l = ffs64(sp);
+        const int js = __builtin_amdgcn_readlane(job, l), cs = __builtin_amdgcn_readlane(c, l);
+        const int ks = __builtin_amdgcn_readlane(key, l);
+        Shape SA, SB;
+        src.shapes_ref(ks, SA, SB);
+        const EpaResult rw = epa_whole(L, epa_shapes_group<true>(SA, SB, lane), qsim[js], np, lane);
+        if (lane == 0) src.epa_result(cs, ks, rw);
+    }
+}
+
+// A lane number that the compiler does not know as threadIdx.x & 63: the wider tiers'
+// lane constants are then worked out where they are used, not kept in registers through
+// the step's other phases (168-register kernels: 45 spilled registers -> 10).
+__device__ __forceinline__ int opaque_lane()
+{
+    int lane = lane_id();
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // Source interface (duck-typed):
 //   int key(int c) const                                 the pair of candidate c, as an int
 //   static constexpr bool kMemCorners                    box corners readable in memory:
@@ -1278,14 +1631,12 @@ __device__ __forceinline__ int gjk_lane_call(GjkLane &G, float *cyc, const Narro
 //   void shapes(int key, Shape &A, Shape &B) const       both shapes of the pair
 //   void gjk_result(int c, int gjk) const                 every candidate
 //   void epa_result(int c, int key, const EpaResult &r) const   every GJK hit (lane 0 calls)
-// ISL: the FP64-islands mode runs the grouped tiers too (their final face choice
-// in binary64); without it, that mode runs every polytope by the whole wave.
+// ISL: the FP64-islands mode (the final face chosen in binary64).
 // The team's wave k uses epa[k]; sh, qidx and qsim are the team's own.
 template <bool ISL = false, class Src>
 __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
                             NarrowShared &sh, int *qidx, SimplexRec *qsim)
 {
-    const bool grouped = ISL || !np.fp64_islands;
     const int lane = lane_id();
     if (team.rank == 0) {
         sh.next = 0;
@@ -1294,8 +1645,7 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
         sh.gjk_done = 0;
         sh.stalled = 0;
     }
-    if (grouped)
-        for (int k = team.rank; k < ncand; k += team.size) qidx[k] = -1;  // queue slots: unpublished
+    for (int k = team.rank; k < ncand; k += team.size) qidx[k] = -1;  // queue slots: unpublished
     team.sync();
     {
         // GJK lanes (gjk_lane_call); the cycle state lives in the wave's EPA LDS,
@@ -1331,28 +1681,26 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
         if (lane == 0) __hip_atomic_fetch_add(&sh.gjk_done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
     EpaLds &L = epa[team.rank >> 6];
-    if (grouped) {
-        // four pairs per wave, one per 16-lane group, started while other waves
-        // may still be in GJK; a spilled polytope is redone by the whole wave
-        const int NW = team.waves();
-        EpgLds<16> &G = *reinterpret_cast<EpgLds<16> *>(&L);
-        const int j = lane & 15;
-        // A pass takes four queue slots, one per group.  The next pass's slots are
-        // claimed while this one starts, their contents loaded (relaxed) under its
-        // work, and then confirmed by an acquire fence, or waited for.
-        auto claim = [&]() {
+    const int NW = team.waves();
+    if (ncand <= EPL_MIN * NW) {
+        // few pairs, whose latency counts: four at a time in 16-lane groups, started while
+        // other waves may still be in GJK.  The next pass's slots are claimed while this
+        // one starts, their contents loaded (relaxed) under its work, and then confirmed
+        // by an acquire fence, or waited for.
+        const int ol = opaque_lane(), j = ol & 15;
+        auto claim = [&]() __attribute__((always_inline)) {
             int b = 0;
-            if (lane == 0) b = atomicAdd(&sh.epa_next, 4);
+            if (ol == 0) b = atomicAdd(&sh.epa_next, 4);
             return __builtin_amdgcn_readfirstlane(b);
         };
-        auto peek = [&](int b) {
-            const int job = b + (lane >> 4);
+        auto peek = [&](int b) __attribute__((always_inline)) {
+            const int job = b + (ol >> 4);
             return job < ncand ? __hip_atomic_load(&qidx[job], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : -1;
         };
-        // the candidate of this group's slot, or -1 once it is certain the slot
-        // stays empty (every wave has left GJK and it was never published)
-        auto resolve = [&](int b, int seen) {
-            const int job = b + (lane >> 4);
+        // the candidate of this group's slot, or -1 once it is certain the slot stays
+        // empty (every wave has left GJK and it was never published)
+        auto resolve = [&](int b, int seen) __attribute__((always_inline)) {
+            const int job = b + (ol >> 4);
             int c = -1;
             if (job < ncand) {
                 if (seen >= 0 && seen < ncand) {
@@ -1360,25 +1708,16 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
                     return seen;
                 }
                 for (int round = 0;; ++round) {
+                    const bool last =
+                        __hip_atomic_load(&sh.gjk_done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == NW;
                     c = __hip_atomic_load(&qidx[job], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    if (c >= ncand) {  // not a candidate of this block: never published here
+                    const bool bad = c >= ncand;  // not a candidate of this block: never published here
+                    if (bad || (c < 0 && !last && round >= EPA_WAIT_ROUNDS)) {
                         if (j == 0) atomicAdd(&sh.stalled, 1);
                         c = -1;
                         break;
                     }
-                    if (c >= 0) break;
-                    if (__hip_atomic_load(&sh.gjk_done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == NW) {
-                        c = __hip_atomic_load(&qidx[job], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                        if (c >= ncand) {
-                            if (j == 0) atomicAdd(&sh.stalled, 1);
-                            c = -1;
-                        }
-                        break;
-                    }
-                    if (round >= EPA_WAIT_ROUNDS) {
-                        if (j == 0) atomicAdd(&sh.stalled, 1);
-                        break;
-                    }
+                    if (c >= 0 || last) break;
                     __builtin_amdgcn_s_sleep(2);
                 }
             }
@@ -1388,118 +1727,134 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
         int c = resolve(base, peek(base));
         for (;;) {
             // slots are filled in order, so an empty first slot ends the queue
-            if (__shfl(c, 0, 64) < 0) break;
-            const int job = base + (lane >> 4);
+            if (__builtin_amdgcn_readlane(c, 0) < 0) break;
             const bool act = c >= 0;
-            const int jq = act ? job : base;
-            if (!act) c = __shfl(c, 0, 64);
-            const int key = qsim[jq].key;
-            Shape A, B;
-            if constexpr (Src::kMemCorners) src.shapes_ref(key, A, B);
-            else src.shapes(key, A, B);
-            const EpaShapes es = epa_shapes_group<Src::kMemCorners>(A, B);
-            V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
-            if (j < 4) {
-                const SimplexRec &q = qsim[jq];
-                sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
-                sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
-            }
-            wave_sync();
-            const int nbase = claim();
-            const int seen = peek(nbase);
-            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np);
-            if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
-            const uint64_t spill = ballot(act && j == 0 && r.status == EPA_SPILL);
-            wave_sync();
-            for (uint64_t sp = spill; sp; sp &= sp - 1) {
-                const int sg = ffs64(sp) >> 4;  // the spilled group
-                const int cs = __shfl(c, 16 * sg, 64);
-                const int ks = __shfl(key, 16 * sg, 64);
-                Shape SA, SB;
-                src.shapes(ks, SA, SB);
-                const EpaShapes ew = epa_shapes(SA, SB);
-                V3 p0 = mk3(0.0f, 0.0f, 0.0f);
-                if (lane < 4) {
-                    const SimplexRec &q = qsim[base + sg];
-                    V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
-                    V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
-                    p0 = sub(a, b);
-                    st3(L.va, lane, a);
-                    st3(L.vb, lane, b);
-                    st3(L.vp, lane, p0);
-                }
-                wave_sync();
-                const EpaResult rw = epa_wave(L, ew, p0, np);
-                if (lane == 0) src.epa_result(cs, ks, rw);
-                wave_sync();
-            }
+            const int c0 = __builtin_amdgcn_readlane(c, 0);
+            int nbase = 0, seen = -1;
+            epa_four<ISL>(src, L, qsim, act ? base + (ol >> 4) : base, act ? c : c0, act, np, ol, [&]() {
+                nbase = claim();
+                seen = peek(nbase);
+            });
             base = nbase;
             c = resolve(base, seen);
         }
         team.sync();
         return;
     }
-    team.sync();
-    const int nepa = sh.nepa;
+    // more: a pair of boxes per lane of EPL_LANES, started as above; a lane takes a queue
+    // slot, waits for it to be published, and goes on to another when its pair is done.
+    // Slots are taken and contacts worked out for EPL_REFILL lanes together.  What
+    // outgrows a lane is chained and runs after the queue's end (inside this loop the
+    // wider tiers' lane constants would live through it), four pairs at a time in 16-lane
+    // groups and then, if it outgrows those, by the whole wave.
+    const uint64_t lower = (1ull << lane) - 1ull;
+    EpaLane e;
+    e.w = reinterpret_cast<float *>(&L) + (lane < EPL_LANES ? lane : 0);
+    int job = -1, c = -1;         // the lane's slot, and its candidate once it runs
+    int st = EPA_NONE;            // of the pair: EPA_NONE while it runs
+    bool out = lane >= EPL_LANES; // no more slots for this lane
+    int chain = -1, rounds = 0;
+    wave_sync();
     for (;;) {
-        int job = 0;
-        if (lane == 0) job = atomicAdd(&sh.epa_next, 1);
-        job = __builtin_amdgcn_readfirstlane(job);
-        if (job >= nepa) break;
-        const int c = qidx[job];
-        const int key = qsim[job].key;
-        Shape A, B;
-        src.shapes(key, A, B);
-        const EpaShapes es = epa_shapes(A, B);
-        V3 p0 = mk3(0.0f, 0.0f, 0.0f);
-        if (lane < 4) {
-            const SimplexRec &q = qsim[job];
-            V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
-            V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
-            p0 = sub(a, b);
-            st3(L.va, lane, a);
-            st3(L.vb, lane, b);
-            st3(L.vp, lane, p0);
+        const uint64_t running = ballot(c >= 0 && st == EPA_NONE);
+        if (!running || __popcll(running) <= EPL_LANES - EPL_REFILL) {
+            // the pairs that are done
+            if (c >= 0 && st != EPA_NONE) {
+                if (st != EPA_SPILL) {
+                    EpaResult r;
+                    if (st == EPA_CONTACT) {
+                        r = epa_lane_finish<ISL>(e, qsim[job].a, qsim[job].b);
+                    } else {
+                        r.pa = r.pb = r.n = mk3(0.0f, 0.0f, 0.0f);
+                        r.depth = 0.0;
+                        r.status = st;
+                    }
+                    src.epa_result(c, qsim[job].key, r);
+                }
+            }
+            for (uint64_t ms = ballot(c >= 0 && st == EPA_SPILL); ms; ms &= ms - 1) {
+                const int js = __builtin_amdgcn_readlane(job, ffs64(ms));
+                if (lane == 0) qsim[js].next = chain;
+                chain = js;
+            }
+            if (c >= 0 && st != EPA_NONE) job = c = -1;
+            // slots for the idle lanes
+            const bool need = job < 0 && !out;
+            const uint64_t m = ballot(need);
+            if (m) {
+                int b = 0;
+                if (lane == 0) b = atomicAdd(&sh.epa_next, __popcll(m));
+                b = __builtin_amdgcn_readfirstlane(b);
+                if (need) job = b + __popcll(m & lower);
+            }
+            // start the pairs whose slots are published; a slot stays empty once every
+            // wave has left GJK without filling it
+            bool wait = job >= 0 && c < 0;
+            if (wait) {
+                const bool last = __hip_atomic_load(&sh.gjk_done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == NW;
+                const int q = job < ncand ? __hip_atomic_load(&qidx[job], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)
+                                          : -1;
+                if (q >= 0 && q < ncand) {
+                    c = q;
+                    Shape A, B;
+                    src.shapes_ref(qsim[job].key, A, B);
+                    e.va = A.vm;
+                    e.vb = B.vm;
+                    st = EPA_SPILL;
+                    if (A.kind == SHAPE_BOX && B.kind == SHAPE_BOX &&
+                        epa_lane_start(e, qsim[job].a, qsim[job].b))
+                        st = EPA_NONE;
+                    wait = false;
+                } else if (q >= ncand || last || job >= ncand) {
+                    if (q >= ncand) atomicAdd(&sh.stalled, 1);
+                    job = -1;
+                    out = true;
+                    wait = false;
+                }
+            }
+            if (!ballot(c >= 0)) {
+                const uint64_t w = ballot(wait);
+                if (!w) {
+                    if (!ballot(!out)) break;
+                    continue;
+                }
+                if (++rounds >= EPA_WAIT_ROUNDS) {
+                    if (lane == 0) atomicAdd(&sh.stalled, __popcll(w));
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(2);
+                continue;
+            }
         }
-        wave_sync();
-        const EpaResult r = epa_wave(L, es, p0, np);
-        if (lane == 0) src.epa_result(c, key, r);
-        wave_sync();
+        if (c >= 0 && st == EPA_NONE) st = epa_lane_trip(e, np);
+    }
+    Team::wave().sync();  // the chain's links
+    const int ol = opaque_lane();
+    while (chain >= 0) {
+        int job = -1;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            if (ol >> 4 == g) job = chain;
+            if (chain >= 0) chain = __builtin_amdgcn_readfirstlane(qsim[chain].next);
+        }
+        const bool act = job >= 0;
+        const int first = __builtin_amdgcn_readlane(job, 0);
+        job = act ? job : first;
+        epa_four<ISL>(src, L, qsim, job, qidx[job], act, np, ol, []() {});
     }
     team.sync();
-}
-
-// EPA of one queued pair by the whole wave: supports of its four simplex vertices
-// in q, every lane returns the result.
-__device__ inline EpaResult epa_whole(EpaLds &L, const EpaShapes &es, const SimplexRec &q, const NarrowParams &np)
-{
-    const int lane = lane_id();
-    V3 p0 = mk3(0.0f, 0.0f, 0.0f);
-    if (lane < 4) {
-        const V3 a = mk3(q.a[3 * lane], q.a[3 * lane + 1], q.a[3 * lane + 2]);
-        const V3 b = mk3(q.b[3 * lane], q.b[3 * lane + 1], q.b[3 * lane + 2]);
-        p0 = sub(a, b);
-        st3(L.va, lane, a);
-        st3(L.vb, lane, b);
-        st3(L.vp, lane, p0);
-    }
-    wave_sync();
-    const EpaResult r = epa_wave(L, es, p0, np);
-    wave_sync();
-    return r;
 }
 
 // The same driver for one wave on its own: CheckCollision over the candidates
 // [0, ncand) of src, with no other wave to wait for.  A GJK hit's simplex goes to
 // sim(c), and the wave lists its hits in list[0, ncand): pairs for the narrow tier
 // from the front, pairs for the wide tier from the back.  The tiers then run over
-// dense lists: four pairs at a time in 16-lane groups, their spills with the wide
-// list two at a time in 32-lane groups (WIDE; else spills go to the whole wave),
-// and what outgrows those by the whole wave.  A wave with one hit gives it to the
+// dense lists: four pairs at a time in 16-lane groups, their spills with the wide list
+// two at a time in 32-lane groups, and what outgrows those by the whole wave.  A wave with one hit gives it to the
 // whole wave at once, and two to the 32-lane tier, since the lanes are idle
 // otherwise and the narrow tiers' attempts would only lengthen the chain.
-template <bool WIDE, bool ISL, class Src>
-__device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list, int &found)
+template <bool ISL, class Src>
+__device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list, int &found)
 {
     const int lane = lane_id();
     const uint64_t lower = (1ull << lane) - 1ull;
@@ -1534,7 +1889,7 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
             }
             // a sphere's support gives a new vertex at every iteration, so its polytopes
             // outgrow a 16-lane group
-            const bool wide = WIDE && hit && (G.A.kind != SHAPE_BOX || G.B.kind != SHAPE_BOX);
+            const bool wide = hit && (G.A.kind != SHAPE_BOX || G.B.kind != SHAPE_BOX);
             const uint64_t mn = ballot(hit && !wide), mw = ballot(wide);
             if (hit) list[wide ? ncand - 1 - nw - __popcll(mw & lower) : nn + __popcll(mn & lower)] = G.c;
             nn += __popcll(mn);
@@ -1560,7 +1915,7 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
     int nspill = 0;  // pairs that outgrew the narrow tier, at list[0, nspill)
     if (nn + nw == 1) {
         nspill = nn;
-    } else if (WIDE && nn + nw == 2) {
+    } else if (nn + nw == 2) {
         nspill = nn;
     } else {
         EpgLds<16> &G = *reinterpret_cast<EpgLds<16> *>(&L);
@@ -1581,7 +1936,7 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
                 sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
             }
             wave_sync();
-            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np);
+            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np, lane);
             if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
             // the spilled pairs move to the front of the list, over entries already read
             const bool sp = act && j == 0 && r.status == EPA_SPILL;
@@ -1602,8 +1957,8 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
         const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np);
         if (lane == 0) src.epa_result(c, key, r);
     };
-    if (!WIDE || nwide == 1) {
-        for (int k = 0; k < nwide; ++k) whole(item(k));
+    if (nwide == 1) {
+        whole(item(0));
     } else {
         EpgLds<32> &G2 = *reinterpret_cast<EpgLds<32> *>(&L);
         const int j = lane & 31;
@@ -1622,7 +1977,7 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
                 sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
             }
             wave_sync();
-            const EpaResult r = epa_group<32, ISL>(G2, es, sa0, sb0, act, np);
+            const EpaResult r = epa_group<32, ISL>(G2, es, sa0, sb0, act, np, lane);
             if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
             uint64_t sp = ballot(act && j == 0 && r.status == EPA_SPILL);
             wave_sync();
@@ -1630,14 +1985,6 @@ __device__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, E
         }
     }
     fence();
-}
-
-// narrow_team by the whole workgroup of BLOCK threads
-template <int BLOCK, bool ISL = false, class Src>
-__device__ inline void narrow_block(const Src &src, int ncand, const NarrowParams &np, EpaLds *epa,
-                                    NarrowShared &sh, int *qidx, SimplexRec *qsim)
-{
-    narrow_team<ISL>(Team::block(BLOCK), src, ncand, np, epa, sh, qidx, qsim);
 }
 
 }  // namespace nans

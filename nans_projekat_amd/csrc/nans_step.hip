@@ -69,7 +69,7 @@ __device__ inline int block_rank(bool pred, int *wave_tot, int &total)
 }
 
 // A body's shape without its corner registers: kind, centre, radius and vm.
-__device__ inline Shape body_shape_ref(const Planes &B, const float *verts, int slot, int nb, const FloorDev &fl)
+__device__ __forceinline__ Shape body_shape_ref(const Planes &B, const float *verts, int slot, int nb, const FloorDev &fl)
 {
     Shape s;
     if (slot < 0) {
@@ -91,7 +91,7 @@ __device__ inline Shape body_shape_ref(const Planes &B, const float *verts, int 
     return s;
 }
 
-__device__ inline Shape body_shape(const Planes &B, const float *verts, int slot, int nb, const FloorDev &fl)
+__device__ __forceinline__ Shape body_shape(const Planes &B, const float *verts, int slot, int nb, const FloorDev &fl)
 {
     Shape s;
     if (slot < 0) {
@@ -148,8 +148,8 @@ struct WorldSrc {
     int *flag;
     unsigned long long *cnt;
     PairDecode32 dec;  // SMALL: the world's decode terms
-    __device__ int key(int c) const { return cand[c]; }
-    __device__ void shapes(int key, Shape &A, Shape &Bs) const
+    __device__ __forceinline__ int key(int c) const { return cand[c]; }
+    __device__ __forceinline__ void shapes(int key, Shape &A, Shape &Bs) const
     {
         PairId q = SMALL ? decode_pair32(key, dec) : decode_pair(key, nb, ns);
         int sa, sb;
@@ -158,7 +158,7 @@ struct WorldSrc {
         Bs = body_shape(B, verts, sb, nb, *fl);
     }
     static constexpr bool kMemCorners = true;
-    __device__ void shapes_ref(int key, Shape &A, Shape &Bs) const
+    __device__ __forceinline__ void shapes_ref(int key, Shape &A, Shape &Bs) const
     {
         PairId q = SMALL ? decode_pair32(key, dec) : decode_pair(key, nb, ns);
         int sa, sb;
@@ -166,8 +166,8 @@ struct WorldSrc {
         A = body_shape_ref(B, verts, sa, nb, *fl);
         Bs = body_shape_ref(B, verts, sb, nb, *fl);
     }
-    __device__ void gjk_result(int c, int g) const { flag[c] = 0; }
-    __device__ void epa_result(int c, int key, const EpaResult &r) const
+    __device__ __forceinline__ void gjk_result(int c, int g) const { flag[c] = 0; }
+    __device__ __forceinline__ void epa_result(int c, int key, const EpaResult &r) const
     {
         if (r.status == EPA_OVERFLOW) atomicAdd(&cnt[CNT_EPA_OVERFLOW], 1ull);
         if (r.status != EPA_CONTACT) return;
@@ -646,8 +646,13 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan(const int *counts, int nb
 #include "nans_broadphase.hpp"
 namespace nans {
 
-constexpr int NARROW_RANGE = 512;  // largest share of candidates per workgroup of the plain narrowphase
+// Shares of candidates per workgroup of the plain narrowphase: 16 to NARROW_RANGE, so
+// that two workgroups per CU get one (shares of at least 64: a 28-body world's
+// narrowphase takes 54 us, with 16 49; 8192 bodies' 46.4, with 16 46.7).
+constexpr int NARROW_RANGE = 512;
+constexpr int NARROW_GRID = 512;
 
+template <bool ISL>
 __global__ __launch_bounds__(256) void k_plain_narrow(Planes B, const float *verts, int nb, int ns,
                                                       const FloorDev *flp, const int *cand, const int *ncand,
                                                       NarrowParams np, ContactRec *rec, int *flag, int *qidx,
@@ -655,16 +660,13 @@ __global__ __launch_bounds__(256) void k_plain_narrow(Planes B, const float *ver
 {
     __shared__ EpaLds lds[4];
     __shared__ NarrowShared sh;
-    __shared__ FloorDev fl;
-    if (threadIdx.x == 0) fl = *flp;
-    __syncthreads();
+    const FloorDev &fl = *flp;  // in global memory, as the box corners
     const int total = *ncand;
-    // shares of 64..NARROW_RANGE candidates, small enough to give every workgroup one
-    const int range = min(NARROW_RANGE, max(64, ((total + (int)gridDim.x - 1) / (int)gridDim.x + 63) & ~63));
+    const int range = min(NARROW_RANGE, max(16, ((total + NARROW_GRID - 1) / NARROW_GRID + 15) & ~15));
     for (int base = blockIdx.x * range; base < total; base += gridDim.x * range) {
         const int count = min(range, total - base);
         WorldSrc<false> src{B, verts, nb, ns, &fl, cand + base, rec + base, flag + base, cnt, PairDecode32{}};
-        narrow_block<256>(src, count, np, lds, sh, qidx + base, qsim + base);
+        narrow_team<ISL>(Team::block(256), src, count, np, lds, sh, qidx + base, qsim + base);
         if (threadIdx.x == 0) {
             atomicAdd(&cnt[CNT_GJK_FOUND], (unsigned long long)sh.nepa);
             if (sh.stalled) atomicAdd(&cnt[CNT_EPA_OVERFLOW], (unsigned long long)sh.stalled);
@@ -1882,8 +1884,9 @@ int nans_step_plain(nans_ctx *ctx, int32_t nsteps)
                     k_plain_cull<true><<<nblk, 256, 0, ls>>>(B, brad, nb, ns, npairs, W->floor, nullptr,
                                                              blk_offsets, cand, W->cand_cap, W->cnt);
                 }
-                int grid = std::max(1, std::min((W->cand_cap + NARROW_RANGE - 1) / NARROW_RANGE, 2048));
-                k_plain_narrow<<<grid, 256, 0, ls>>>(B, verts, nb, ns, W->floor, cand, ncand, k.np, rec, flag,
+                const int grid = std::max(1, std::min((W->cand_cap + 15) / 16, NARROW_GRID));
+                auto narrow = k.np.fp64_islands ? k_plain_narrow<true> : k_plain_narrow<false>;
+                narrow<<<grid, 256, 0, ls>>>(B, verts, nb, ns, W->floor, cand, ncand, k.np, rec, flag,
                                                      qidx, qsim, W->cnt);
             } else {
                 k_zero_i32<<<1, 64, 0, ls>>>(ncand, 1);

@@ -120,7 +120,7 @@ __host__ __device__ inline void integrate_velocities_quat(const Planes &B, const
 
 // Corners of a box Model (UpdateVertices, code/nans.cpp:394-407) and the
 // bounding radius max |v - P| used by the cull.
-__device__ inline float box_vertices_model(const M4 &m, V3 P, float *out24)
+__device__ __forceinline__ float box_vertices_model(const M4 &m, V3 P, float *out24)
 {
     V3 v[8];
     model_vertices(m, v);
@@ -142,13 +142,13 @@ __device__ inline float box_vertices_model(const M4 &m, V3 P, float *out24)
 
 // Box corners of the Model rebuilt from the pose (code/nans.cpp:1913-1941), or in
 // the quaternion mode from the quaternion planes of Q.
-__device__ inline float box_vertices_body(const Planes &B, int i, float *out24)
+__device__ __forceinline__ float box_vertices_body(const Planes &B, int i, float *out24)
 {
     const V3 P = B.get3(F_PX, i);
     return box_vertices_model(model_from_pose(P, B.get3(F_AX, i), B.get3(F_SX, i)), P, out24);
 }
 
-__device__ inline float box_vertices_quat(const Planes &B, const Planes &Q, int i, float *out24)
+__device__ __forceinline__ float box_vertices_quat(const Planes &B, const Planes &Q, int i, float *out24)
 {
     const V3 P = B.get3(F_PX, i);
     return box_vertices_model(
@@ -168,7 +168,7 @@ __host__ __device__ inline int64_t pair_count(int nb, int ns)
 }
 
 // Row i of the upper triangle (i < j) holding linear index p; row i starts at i*(2n-i-1)/2.
-__device__ inline void tri_decode(int64_t p, int n, int &i, int &j)
+__device__ __forceinline__ void tri_decode(int64_t p, int n, int &i, int &j)
 {
     // a binary32 estimate of the row; the two loops below make it exact
     const float b = 2.0f * (float)n - 1.0f;
@@ -182,7 +182,7 @@ __device__ inline void tri_decode(int64_t p, int n, int &i, int &j)
 }
 
 // Canonical pair p of a world: CC(i<j), CF(i), SF(s), CS(cube-major), SS(s<t).
-__device__ inline PairId decode_pair(int64_t p, int nb, int ns)
+__device__ __forceinline__ PairId decode_pair(int64_t p, int nb, int ns)
 {
     PairId q;
     int64_t ncc = tri(nb);
@@ -250,7 +250,7 @@ __device__ inline PairDecode32 pair_decode32(int nb, int ns)
 }
 
 // b = 2n - 1 and bb = b * b as binary32
-__device__ inline void tri_decode32(int p, int n, float b, float bb, int &i, int &j)
+__device__ __forceinline__ void tri_decode32(int p, int n, float b, float bb, int &i, int &j)
 {
     const float disc = bb - 8.0f * (float)p;
     int r = (int)((b - __builtin_amdgcn_sqrtf(disc > 0.0f ? disc : 0.0f)) * 0.5f);
@@ -262,7 +262,7 @@ __device__ inline void tri_decode32(int p, int n, float b, float bb, int &i, int
     j = p - start(r) + r + 1;
 }
 
-__device__ inline PairId decode_pair32(int p, const PairDecode32 &d)
+__device__ __forceinline__ PairId decode_pair32(int p, const PairDecode32 &d)
 {
     const int nb = d.nb, ns = d.ns;
     PairId q;
