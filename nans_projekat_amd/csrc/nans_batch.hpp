@@ -25,7 +25,8 @@ constexpr size_t plain_small_fixed_bytes(int n)
 {
     return sizeof(int) * ((size_t)(3 + F_NLDS) * ((n + 3) & ~3) + 4);
 }
-constexpr int CULL_CHUNK = 4096;          // canonical pairs per block of the plain cull
+constexpr int CULL_CHUNK = 4096;          // canonical pairs per block of the plain cull at most,
+constexpr int CULL_BLOCKS = 512;          // fewer where this many blocks then suffice
 
 enum : int {
     CNT_EPA_OVERFLOW = 0,
