@@ -149,6 +149,7 @@ struct nans_worlds {
     int64_t max_pairs = 0;
     std::vector<int> h_off, h_nb;
     std::vector<float> h_fric, h_rest;
+    std::vector<float> quat_angles;  // nans_set_state's angles while their quaternions are not made
     float *planes = nullptr;
     float *verts = nullptr;
     float *brad = nullptr;
