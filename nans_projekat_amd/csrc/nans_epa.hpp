@@ -1,7 +1,8 @@
 // nans_epa.hpp -- EPA (ResolveCollision, code/nans.cpp:787-904) by one wavefront
-// per pair, and the workgroup narrowphase driver (GJK per lane, EPA per wave).
+// per pair, by groups of 16 or 32 lanes and by single lanes, and the narrowphase
+// drivers (GJK per lane, then EPA) of a workgroup and of a wave.
 //
-// Layout of the polytope:
+// Layout of the whole wave's polytope:
 //   vertices   registers: lane l holds vertex l (and lane l < 8 vertex 64 + l): its
 //              P and its equality class (the first vertex with the same P, 255 if
 //              P has a NaN: never equal); LDS keeps P, SupA, SupB for gathers;
@@ -1423,12 +1424,12 @@ __device__ __forceinline__ EpaResult epa_lane_finish(const EpaLane &e, const flo
 //        have ended take the next candidates together once GJK_REFILL_MIN of
 //        them wait (work is handed out per wave by one LDS atomic), so a wave is
 //        not held by its slowest lane;
-//   EPA  the GJK hits are queued with their simplex; each wave takes queued hits
-//        (LDS atomic) and runs ResolveCollision on them with the polytope in its
-//        LDS block.  In the reference's arithmetic a wave starts on the queue as
+//   EPA  the GJK hits are queued with their simplex; the waves take queued hits (LDS
+//        atomic) and run ResolveCollision on them, a pair per lane or four per wave,
+//        with the polytopes in the wave's LDS block.  A wave starts on the queue as
 //        soon as its own GJK lanes are done, while other waves still run GJK: a
 //        hit's queue slot is published with a release store of its candidate
-//        index, and a wave that takes a slot not yet published waits for it, or
+//        index, and a lane that takes a slot not yet published waits for it, or
 //        for every wave to leave GJK (then the slot will never be filled).
 // Results go through the source object, per candidate, so their order is that
 // of the candidates whatever the order of the work.
