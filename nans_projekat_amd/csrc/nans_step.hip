@@ -2453,14 +2453,22 @@ int nans_set_state(nans_ctx *ctx, const nans_bodies_soa *b)
     // binary64 on the host)
     W->quat_angles.assign(b->angles, b->angles + 3 * N);
     if (ctx->orientation == NANS_ORIENT_QUATERNION) NANS_TRY(settle_quaternions(W));
-    return warm_reset(ctx);
+    NANS_TRY(warm_reset(ctx));
+    // the next call may be on another stream: the zeroing kernels end here
+    NANS_HIP(hipGetLastError());
+    NANS_HIP(hipStreamSynchronize(ctx->stream));
+    return NANS_OK;
 }
 
 int nans_set_warm_start(nans_ctx *ctx, int32_t enable)
 {
     NANS_REQUIRE(ctx, NANS_ERR_INVALID, "ctx is NULL");
     NANS_REQUIRE(enable == 0 || enable == 1, NANS_ERR_INVALID, "enable must be 0 or 1");
-    if (enable && !ctx->warm) NANS_TRY(warm_reset(ctx));
+    if (enable && !ctx->warm) {
+        NANS_HIP(hipSetDevice(ctx->p.device));
+        NANS_TRY(warm_reset(ctx));
+        NANS_HIP(hipStreamSynchronize(ctx->stream));  // as nans_set_state's
+    }
     ctx->warm = enable;
     return NANS_OK;
 }
