@@ -66,9 +66,7 @@ struct PairSrc {
     unsigned long long *overflow;
     SimplexRec *simplex;
     __device__ SimplexRec &sim(int c) const { return simplex[c]; }
-    static constexpr bool kMemCorners = false;
     __device__ int key(int c) const { return c; }
-    __device__ void shapes_ref(int key, Shape &A, Shape &B) const { shapes(key, A, B); }
     __device__ void shapes(int key, Shape &A, Shape &B) const
     {
         A = load_shape(a, base + key, n);
@@ -106,7 +104,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PE
 {
     __shared__ EpaLds lds[4];
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    int found = 0;
     for (;;) {
         unsigned long long t = 0;
         wave_sync();  // the wave meets on both sides of the claim
@@ -118,7 +115,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PE
         if (base >= n) break;
         const int count = (int)min((int64_t)share, n - base);
         PairSrc src{a, b, base, n, o, &cnt[0], sim + base};
-        narrow_wave<ISL>(src, count, p, lds[wv], list + base, found);
+        narrow_wave<ISL>(src, count, p, lds[wv], list + base);
     }
 }
 

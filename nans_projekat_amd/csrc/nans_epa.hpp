@@ -1626,10 +1626,9 @@ __device__ __forceinline__ int opaque_lane()
 
 // Source interface (duck-typed):
 //   int key(int c) const                                 the pair of candidate c, as an int
-//   static constexpr bool kMemCorners                    box corners readable in memory:
-//   void shapes_ref(int key, Shape &A, Shape &B) const   then both shapes of the pair
-//                                                        with Shape::vm and no v[]
 //   void shapes(int key, Shape &A, Shape &B) const       both shapes of the pair
+//   void shapes_ref(int key, Shape &A, Shape &B) const   the same with Shape::vm (box corners in
+//                                                        memory) and no v[]
 //   void gjk_result(int c, int gjk) const                 every candidate
 //   void epa_result(int c, int key, const EpaResult &r) const   every GJK hit (lane 0 calls)
 // ISL: the FP64-islands mode (the final face chosen in binary64).
@@ -1851,11 +1850,13 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
 // sim(c), and the wave lists its hits in list[0, ncand): pairs for the narrow tier
 // from the front, pairs for the wide tier from the back.  The tiers then run over
 // dense lists: four pairs at a time in 16-lane groups, their spills with the wide list
-// two at a time in 32-lane groups, and what outgrows those by the whole wave.  A wave with one hit gives it to the
-// whole wave at once, and two to the 32-lane tier, since the lanes are idle
-// otherwise and the narrow tiers' attempts would only lengthen the chain.
+// two at a time in 32-lane groups, and what outgrows those by the whole wave.  A wave
+// with one hit gives it to the whole wave at once, and two to the 32-lane tier, since
+// the lanes are idle otherwise and the narrow tiers' attempts would only lengthen the
+// chain.  The tiers see an opaque lane (25 spilled registers -> 2; 777 pairs 137 -> 124
+// us, 200k 1.06 -> 1.04 ms).
 template <bool ISL, class Src>
-__device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list, int &found)
+__device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list)
 {
     const int lane = lane_id();
     const uint64_t lower = (1ull << lane) - 1ull;
@@ -1898,51 +1899,34 @@ __device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const Nar
             if (g != GJK_STILL) G.c = -1;
         }
     }
-    found += nn + nw;
     fence();
-    if (!ISL && np.fp64_islands) {  // the grouped tiers' islands choice is the ISL instantiation's
-        for (int k = 0; k < nn + nw; ++k) {
-            const int c = list[k < nn ? k : ncand - 1 - (k - nn)];
-            const SimplexRec &q = src.sim(c);
-            const int key = q.key;
-            Shape A, B;
-            src.shapes(key, A, B);
-            const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np);
-            if (lane == 0) src.epa_result(c, key, r);
-        }
-        fence();
-        return;
-    }
     int nspill = 0;  // pairs that outgrew the narrow tier, at list[0, nspill)
-    if (nn + nw == 1) {
-        nspill = nn;
-    } else if (nn + nw == 2) {
+    if (nn + nw <= 2) {
         nspill = nn;
     } else {
         EpgLds<16> &G = *reinterpret_cast<EpgLds<16> *>(&L);
-        const int j = lane & 15;
+        const int ol = opaque_lane(), j = ol & 15;
         for (int base = 0; base < nn; base += 4) {
-            const int k = base + (lane >> 4);
+            const int k = base + (ol >> 4);
             const bool act = k < nn;
             const int c = list[act ? k : base];
             const SimplexRec &q = src.sim(c);
             const int key = q.key;
             Shape A, B;
-            if constexpr (Src::kMemCorners) src.shapes_ref(key, A, B);
-            else src.shapes(key, A, B);
-            const EpaShapes es = epa_shapes_group<Src::kMemCorners>(A, B);
+            src.shapes(key, A, B);
+            const EpaShapes es = epa_shapes_group(A, B, ol);
             V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
             if (j < 4) {
                 sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
                 sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
             }
             wave_sync();
-            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np, lane);
+            const EpaResult r = epa_group<16, ISL>(G, es, sa0, sb0, act, np, ol);
             if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
             // the spilled pairs move to the front of the list, over entries already read
             const bool sp = act && j == 0 && r.status == EPA_SPILL;
             const uint64_t ms = ballot(sp);
-            if (sp) list[nspill + __popcll(ms & lower)] = c;
+            if (sp) list[nspill + __popcll(ms & ((1ull << ol) - 1ull))] = c;
             nspill += __popcll(ms);
         }
         fence();
@@ -1950,39 +1934,38 @@ __device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const Nar
     // the wide tiers over the spills, then the wide list
     const int nwide = nspill + nw;
     auto item = [&](int k) { return list[k < nspill ? k : ncand - 1 - (k - nspill)]; };
-    auto whole = [&](int c) {
-        const SimplexRec &q = src.sim(c);
-        const int key = q.key;
-        Shape A, B;
-        src.shapes(key, A, B);
-        const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np);
-        if (lane == 0) src.epa_result(c, key, r);
-    };
-    if (nwide == 1) {
-        whole(item(0));
-    } else {
-        EpgLds<32> &G2 = *reinterpret_cast<EpgLds<32> *>(&L);
-        const int j = lane & 31;
-        for (int base = 0; base < nwide; base += 2) {
-            const int k = base + (lane >> 5);
-            const bool act = k < nwide;
-            const int c = item(act ? k : base);
+    EpgLds<32> &G2 = *reinterpret_cast<EpgLds<32> *>(&L);
+    const int wl = opaque_lane(), jw = wl & 31;
+    for (int base = 0; base < nwide; base += 2) {
+        const int k = base + (wl >> 5);
+        const bool act = k < nwide;
+        const int c = item(act ? k : base);
+        uint64_t sp = 1;  // a pair on its own goes to the whole wave
+        if (nwide > 1) {
             const SimplexRec &q = src.sim(c);
             const int key = q.key;
             Shape A, B;
             src.shapes(key, A, B);
-            const EpaShapes es = epa_shapes_group(A, B);
+            const EpaShapes es = epa_shapes_group(A, B, wl);
             V3 sa0 = mk3(0.0f, 0.0f, 0.0f), sb0 = sa0;
-            if (j < 4) {
-                sa0 = mk3(q.a[3 * j], q.a[3 * j + 1], q.a[3 * j + 2]);
-                sb0 = mk3(q.b[3 * j], q.b[3 * j + 1], q.b[3 * j + 2]);
+            if (jw < 4) {
+                sa0 = mk3(q.a[3 * jw], q.a[3 * jw + 1], q.a[3 * jw + 2]);
+                sb0 = mk3(q.b[3 * jw], q.b[3 * jw + 1], q.b[3 * jw + 2]);
             }
             wave_sync();
-            const EpaResult r = epa_group<32, ISL>(G2, es, sa0, sb0, act, np, lane);
-            if (act && j == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
-            uint64_t sp = ballot(act && j == 0 && r.status == EPA_SPILL);
+            const EpaResult r = epa_group<32, ISL>(G2, es, sa0, sb0, act, np, wl);
+            if (act && jw == 0 && r.status != EPA_SPILL) src.epa_result(c, key, r);
+            sp = ballot(act && jw == 0 && r.status == EPA_SPILL);
             wave_sync();
-            for (; sp; sp &= sp - 1) whole(__builtin_amdgcn_readlane(c, ffs64(sp)));
+        }
+        for (; sp; sp &= sp - 1) {
+            const int cw = __builtin_amdgcn_readlane(c, ffs64(sp));
+            const SimplexRec &q = src.sim(cw);
+            const int key = q.key;
+            Shape A, B;
+            src.shapes(key, A, B);
+            const EpaResult r = epa_whole(L, epa_shapes(A, B), q, np, wl);
+            if (wl == 0) src.epa_result(cw, key, r);
         }
     }
     fence();

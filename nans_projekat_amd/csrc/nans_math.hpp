@@ -184,10 +184,10 @@ __device__ inline M4 model_from_quat(V3 pos, float w, float x, float y, float z,
     return m;
 }
 
-// Model of a box from (centre, unit quaternion (w,x,y,z), half-extents): columns
-// R(q)[:,k] * (2 h_k) and (c, 1).  Used by the narrowphase entry point, whose shapes
-// carry quaternions.
-__device__ inline M4 model_from_box(V3 c, float qw, float qx, float qy, float qz, V3 h)
+// Box corners from (centre, unit quaternion (w,x,y,z), half-extents): Model columns
+// R(q)[:,k] * (2 h_k) and (c, 1), applied with the glm mat4*vec4 form.  Used by the
+// narrowphase entry point, whose shapes carry quaternions.
+__device__ inline void box_from_quat(V3 c, float qw, float qx, float qy, float qz, V3 h, V3 *verts)
 {
     float xx = qx * qx, yy = qy * qy, zz = qz * qz;
     float xy = qx * qy, xz = qx * qz, yz = qy * qz;
@@ -201,13 +201,7 @@ __device__ inline M4 model_from_box(V3 c, float qw, float qx, float qy, float qz
     m.m[4] = r01 * sy; m.m[5] = r11 * sy; m.m[6] = r21 * sy; m.m[7] = 0.0f;
     m.m[8] = r02 * sz; m.m[9] = r12 * sz; m.m[10] = r22 * sz; m.m[11] = 0.0f;
     m.m[12] = c.x; m.m[13] = c.y; m.m[14] = c.z; m.m[15] = 1.0f;
-    return m;
-}
-
-// Its corners, with the glm mat4*vec4 form.
-__device__ inline void box_from_quat(V3 c, float qw, float qx, float qy, float qz, V3 h, V3 *verts)
-{
-    model_vertices(model_from_box(c, qw, qx, qy, qz, h), verts);
+    model_vertices(m, verts);
 }
 
 }  // namespace nans

@@ -157,7 +157,6 @@ struct WorldSrc {
         A = body_shape(B, verts, sa, nb, *fl);
         Bs = body_shape(B, verts, sb, nb, *fl);
     }
-    static constexpr bool kMemCorners = true;
     __device__ __forceinline__ void shapes_ref(int key, Shape &A, Shape &Bs) const
     {
         PairId q = SMALL ? decode_pair32(key, dec) : decode_pair(key, nb, ns);
