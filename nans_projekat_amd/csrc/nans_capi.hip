@@ -58,64 +58,96 @@ __device__ inline void write_pair(const NarrowOutDev &o, int64_t i, int64_t n, i
     if (o.depth) o.depth[i] = depth;
 }
 
-// Candidates of one wave: pairs [base, base + count) of the input arrays.
+// Candidates of one wave: pairs [first, first + count) of its group's (pair()).
 struct PairSrc {
     NarrowIn a, b;
-    int64_t base, n;
+    int64_t first, n;
+    int groups, group, shift;
     NarrowOutDev o;
     unsigned long long *overflow;
     SimplexRec *simplex;
     __device__ SimplexRec &sim(int c) const { return simplex[c]; }
     __device__ int key(int c) const { return c; }
+    // shares of 2^shift pairs go to the groups in turn
+    __device__ int64_t pair(int c) const
+    {
+        const int64_t u = first + c, s = u >> shift;
+        return ((s * groups + group) << shift) + (u - (s << shift));
+    }
     __device__ void shapes(int key, Shape &A, Shape &B) const
     {
-        A = load_shape(a, base + key, n);
-        B = load_shape(b, base + key, n);
+        const int64_t i = pair(key);
+        A = load_shape(a, i, n);
+        B = load_shape(b, i, n);
     }
     __device__ void gjk_result(int c, int g) const
     {
         const V3 z = mk3(0.0f, 0.0f, 0.0f);
-        write_pair(o, base + c, n, g, EPA_NONE, z, z, z, 0.0);
+        write_pair(o, pair(c), n, g, EPA_NONE, z, z, z, 0.0);
     }
     __device__ void epa_result(int c, int key, const EpaResult &r) const
     {
-        write_pair(o, base + c, n, GJK_FOUND, r.status, r.n, r.pa, r.pb, r.depth);
+        write_pair(o, pair(c), n, GJK_FOUND, r.status, r.n, r.pa, r.pb, r.depth);
         if (r.status == EPA_OVERFLOW) atomicAdd(overflow, 1ull);
     }
 };
 
-// The narrowphase entry point: every wave takes a share of the pairs on its own
+// The narrowphase entry point: every wave takes shares of the pairs on its own
 // (narrow_wave), so a small call is spread over the whole chip and no wave waits
-// for the slowest pair of its workgroup.  With 256 pairs per workgroup, 777 pairs
-// ran on four workgroups as a chain of EPA passes (756 us a call, now 136), 30011
-// on 117 of the chip's 256 CUs (942 us, now 440); 1M pairs 4.70 -> 4.03 ms.
-// Shares of at most 32 pairs, so that the last ones end together (1M pairs at 16,
-// 32, 64: 4.10, 3.90, 3.96 ms; 200k in the islands mode 1.19, 1.24, 1.36 ms), and
-// of a quarter of a wave's part of a smaller call, down to one pair.  Three waves
-// per SIMD (168 VGPRs; two take 5.37 ms where three take 4.82, four spill).
+// for the slowest pair of its workgroup.  With 256 pairs per workgroup, 777 random
+// pairs ran on four workgroups as a chain of EPA passes (716 us a call, now 123),
+// 30011 on 117 of the chip's 256 CUs (859 us, now 306); 1M pairs 4.62 -> 3.68 ms.
+// A share is a power of two: a quarter of a wave's part of the call, down to one
+// pair, and at most 32, so that the last ones end together (1M pairs at 16, 32, 64:
+// 4.10, 3.90, 3.96 ms; 200k in the islands mode 1.19, 1.24, 1.36 ms).  Three waves per
+// SIMD (168 VGPRs; two take 5.37 ms where three take 4.82).
 constexpr int NP_SHARE = 32;
 constexpr int NP_WAVES_PER_CU = 12;
+// The shares go in turn to as many groups of workgroups, each of which hands out its
+// own from a counter in its own 128-byte line; a wave's first share is its place in
+// the group, without a claim.  One counter for all serialised the claims at some 15 ns
+// each, and a call whose pairs mostly miss is nothing but claims: pairs that all miss,
+// 30011 / 200k / 1M a call, 249 / 219 / 445 us, now 59 / 47 / 69 (8, 16, 32, 64 groups
+// alike within 5 %).
+constexpr int NP_GROUPS = 32;
+constexpr int NP_CNT_STRIDE = 16;
+constexpr int NP_CNT_WORDS = NP_CNT_STRIDE * (1 + NP_GROUPS);  // [0]: the overflow count
+// A wave that has seen this many pairs in a row miss takes twice as many with its next
+// claim, up to 64, until a pair hits: one share fills few lanes of GJK, and only hits
+// make a share long (all miss, 200k / 1M: 60 / 101 -> 47 / 69 us; at 32 in a row 52 / 69;
+// at 8, 60000 pairs with 1 % overlaps take 154 us instead of 132).
+constexpr int NP_RUN = 16;
 
 // ISL: the FP64-islands mode (grouped EPA tiers with a binary64 final face).
 template <bool ISL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PER_CU / 4))) void k_narrowphase(
-    int64_t n, int share, NarrowIn a, NarrowIn b, NarrowParams p, NarrowOutDev o, unsigned long long *cnt, int *list,
+    int64_t n, int shift, NarrowIn a, NarrowIn b, NarrowParams p, NarrowOutDev o, unsigned long long *cnt, int *list,
     SimplexRec *sim)
 {
     __shared__ EpaLds lds[4];
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    for (;;) {
-        unsigned long long t = 0;
+    const int groups = min(NP_GROUPS, (int)gridDim.x);
+    const int g = (int)blockIdx.x % groups;
+    const int waves = 4 * (((int)gridDim.x - g + groups - 1) / groups);  // of this group
+    // the group's pairs, and how many the groups before it have
+    const int64_t cycle = (int64_t)groups << shift, q = n / cycle, r = n - q * cycle;
+    const int64_t mine = (q << shift) + min((int64_t)1 << shift, max((int64_t)0, r - ((int64_t)g << shift)));
+    const int64_t before = (q << shift) * g + min(r, (int64_t)g << shift);
+    const int64_t started = (int64_t)waves << shift;
+    int take = 1 << shift, run = 0;
+    int64_t first = (int64_t)(4 * ((int)blockIdx.x / groups) + wv) << shift;  // a wave's first share is its own
+    while (first < mine) {
+        const int count = (int)min((int64_t)take, mine - first);
+        PairSrc src{a, b, first, n, groups, g, shift, o, &cnt[0], sim + before + first};
+        run = narrow_wave<ISL>(src, count, p, lds[wv], list + before + first) ? 0 : run + count;
+        if (started >= mine) break;  // the first shares were all
+        take = run >= NP_RUN ? min(64, 2 * take) : 1 << shift;
+        unsigned long long c = 0;
         wave_sync();  // the wave meets on both sides of the claim
-        if (lane_id() == 0) t = atomicAdd(&cnt[1], 1ull);
+        if (lane_id() == 0) c = atomicAdd(&cnt[NP_CNT_STRIDE * (1 + g)], (unsigned long long)take);
         wave_sync();
-        t = ((unsigned long long)__builtin_amdgcn_readfirstlane((int)(t >> 32)) << 32) |
-            (unsigned)__builtin_amdgcn_readfirstlane((int)t);
-        const int64_t base = (int64_t)t * share;
-        if (base >= n) break;
-        const int count = (int)min((int64_t)share, n - base);
-        PairSrc src{a, b, base, n, o, &cnt[0], sim + base};
-        narrow_wave<ISL>(src, count, p, lds[wv], list + base);
+        first = started + (int64_t)(((unsigned long long)__builtin_amdgcn_readfirstlane((int)(c >> 32)) << 32) |
+                                    (unsigned)__builtin_amdgcn_readfirstlane((int)c));
     }
 }
 
@@ -126,10 +158,10 @@ __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v)
 }
 
 // Scratch of nans_narrowphase_noalloc, one copy per device for the life of the
-// process: the EPA overflow counter (in its own 256-byte slot), then the EPA queue
-// of k_narrowphase -- a candidate index and a GJK simplex per pair -- for up to
-// NANS_NARROWPHASE_NOALLOC_MAX_PAIRS pairs (26 MiB in all).
-constexpr size_t NA_CNT_BYTES = 256;
+// process: k_narrowphase's counters, then its hit list -- a candidate index and a GJK
+// simplex per pair -- for up to NANS_NARROWPHASE_NOALLOC_MAX_PAIRS pairs (27 MiB in
+// all).
+constexpr size_t NA_CNT_BYTES = (sizeof(unsigned long long) * NP_CNT_WORDS + 255) / 256 * 256;
 constexpr size_t NA_QIDX_BYTES = sizeof(int) * (size_t)NANS_NARROWPHASE_NOALLOC_MAX_PAIRS;
 constexpr size_t NA_QSIM_BYTES = sizeof(SimplexRec) * (size_t)NANS_NARROWPHASE_NOALLOC_MAX_PAIRS;
 constexpr size_t NA_BYTES = NA_CNT_BYTES + NA_QIDX_BYTES + NA_QSIM_BYTES;
@@ -233,7 +265,7 @@ int nans_create(nans_ctx **out, const nans_params *p)
         delete c;
         return rc;
     }
-    hipError_t e = hipMalloc((void **)&c->d_counters, 64 * sizeof(unsigned long long));
+    hipError_t e = hipMalloc((void **)&c->d_counters, NP_CNT_WORDS * sizeof(unsigned long long));
     if (e != hipSuccess) {
         delete c;
         set_error("hipMalloc: %s", hipGetErrorString(e));
@@ -305,7 +337,7 @@ static int narrow_launch(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, con
                          int64_t *n_overflow)
 {
     hipStream_t s = ctx->stream;
-    k_fill_u64<<<1, 64, 0, s>>>(cnt, 2, 0ull);  // the overflow count, and the next share
+    k_fill_u64<<<(NP_CNT_WORDS + 255) / 256, 256, 0, s>>>(cnt, NP_CNT_WORDS, 0ull);
     NANS_HIP(hipGetLastError());
     if (n > 0) {
         NarrowIn ia{a->type, a->pos, a->quat, a->half};
@@ -314,13 +346,15 @@ static int narrow_launch(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, con
         int cus = 0;
         NANS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->p.device));
         const int64_t waves = NP_WAVES_PER_CU * (int64_t)cus;
-        const int share = (int)std::min<int64_t>(NP_SHARE, std::max<int64_t>(1, n / (4 * waves)));
-        const unsigned grid = (unsigned)std::min<int64_t>((n + 4 * share - 1) / (4 * share), waves / 4);
+        int shift = 0;  // of a share
+        while (2 << shift <= NP_SHARE && (2 << shift) * 4 * waves <= n) ++shift;
+        const int64_t shares = (n + (1 << shift) - 1) >> shift;
+        const unsigned grid = (unsigned)std::min<int64_t>((shares + 3) / 4, waves / 4);
         const NarrowParams np = narrow_params(ctx->p);
         if (ctx->p.fp64_islands)
-            k_narrowphase<true><<<grid, 256, 0, s>>>(n, share, ia, ib, np, o, cnt, qidx, qsim);
+            k_narrowphase<true><<<grid, 256, 0, s>>>(n, shift, ia, ib, np, o, cnt, qidx, qsim);
         else
-            k_narrowphase<false><<<grid, 256, 0, s>>>(n, share, ia, ib, np, o, cnt, qidx, qsim);
+            k_narrowphase<false><<<grid, 256, 0, s>>>(n, shift, ia, ib, np, o, cnt, qidx, qsim);
         NANS_HIP(hipGetLastError());
     }
     unsigned long long ov = 0;

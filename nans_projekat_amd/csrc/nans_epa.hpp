@@ -1854,9 +1854,9 @@ __device__ __forceinline__ void narrow_team(const Team &team, const Src &src, in
 // with one hit gives it to the whole wave at once, and two to the 32-lane tier, since
 // the lanes are idle otherwise and the narrow tiers' attempts would only lengthen the
 // chain.  The tiers see an opaque lane (25 spilled registers -> 2; 777 pairs 137 -> 124
-// us, 200k 1.06 -> 1.04 ms).
+// us, 200k 1.06 -> 1.04 ms).  Returns whether a pair hit.
 template <bool ISL, class Src>
-__device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list)
+__device__ __forceinline__ bool narrow_wave(const Src &src, int ncand, const NarrowParams &np, EpaLds &L, int *list)
 {
     const int lane = lane_id();
     const uint64_t lower = (1ull << lane) - 1ull;
@@ -1969,6 +1969,7 @@ __device__ __forceinline__ void narrow_wave(const Src &src, int ncand, const Nar
         }
     }
     fence();
+    return nn + nw != 0;
 }
 
 }  // namespace nans
