@@ -1,4 +1,5 @@
-"""Worlds of many overlapping bodies, bit for bit against the oracle: boxes mixed with
+"""Worlds of many overlapping bodies, bit for bit against the oracle: contact lists longer
+than the solver's store of terms, which are then solved in parts, and boxes mixed with
 spheres, whose pairs leave the lanes' EPA by different ways (nans_epa.hpp)."""
 import numpy as np
 import pytest
@@ -10,8 +11,20 @@ from test_step_gpu import _state_equal
 
 pytestmark = pytest.mark.gpu
 
+Z3, Z = np.zeros((0, 3), np.float32), np.zeros(0, np.float32)
+
+
 def _params():
     return S.StepParams(dt=1.0 / 120.0, solver_iterations=10, restitution=0.2, friction=0.5)
+
+
+def _heap(n, spread, seed):
+    """Unit cubes whose centres lie in a small cube: (almost) every pair touches."""
+    r = np.random.default_rng(seed)
+    pos = (np.array([2.0, 3.0, 2.0]) + r.uniform(-spread, spread, (n, 3))).astype(np.float32)
+    sc = S._world(pos, np.ones((n, 3), np.float32), np.ones(n, np.float32), Z3, Z3, Z, Z)
+    sc.params = _params()
+    return sc
 
 
 def _mixed(nbox, nsph, seed):
@@ -23,6 +36,44 @@ def _mixed(nbox, nsph, seed):
     sc.angles[:nbox] = r.uniform(-180.0, 180.0, (nbox, 3)).astype(np.float32)
     sc.params = _params()
     return sc
+
+
+# Bytes of a contact's terms (35 words), and an upper bound of the terms a step has room
+# for: all of a CU's LDS in the plain step; in the batched one the radii and polytopes (12 KB
+# a wave at most), and two fifths of a contact record per candidate in scratch.
+TERMS = 140
+
+
+def _room(path, n, npairs, threads):
+    if path == "plain":
+        return 160 * 1024 // TERMS
+    return (4 * n + 12 * 1024 * max(threads, 64) // 64) // TERMS + 2 * npairs // 5
+
+
+@pytest.mark.parametrize("warm", [False, True])
+@pytest.mark.parametrize("path,threads", [("plain", 0), ("batched", 64), ("batched", 256)])
+def test_contact_lists_solved_in_parts(oracle_mod, path, threads, warm):
+    n = 72
+    sc = _heap(n, 0.22, 11)
+    ctx = runtime.Context(sc.params)
+    ctx.upload(sc)
+    ctx.set_batched_block(threads)
+    ctx.set_warm_start(warm)
+    ws = oracle_mod.WorldState(sc, 0, "f32")
+    if warm:
+        ws.enable_warm(16 * n + 64)
+    npairs = n * (n - 1) // 2 + n
+    longest = 0
+    for k in range(4):
+        before = ctx.stats()["contacts"]
+        (ctx.step_plain if path == "plain" else ctx.step_batched)(1)
+        ref = ws.run(1, contacts=True)
+        count = ctx.stats()["contacts"] - before
+        assert count == len(ref)
+        longest = max(longest, count)
+        _state_equal(ctx.download(), ws, 0, n, "%s step %d" % (path, k))
+    assert longest > _room(path, n, npairs, threads)
+    ctx.close()
 
 
 @pytest.mark.parametrize("islands", [0, 1])
