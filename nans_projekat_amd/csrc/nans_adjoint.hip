@@ -26,11 +26,22 @@
 
 namespace nans {
 
-enum : int { ADJ_CNT_OVERFLOW = 0, ADJ_CNT_REPLAY, ADJ_CNT_N };
+// World-steps with more contacts than are kept; whose replay differs from the kept state;
+// whose kept state and replay are both not a number.  Of the last two the first one, as the
+// complement of step << 32 | world (a maximum, so that zero means none).
+enum : int {
+    ADJ_CNT_OVERFLOW = 0,
+    ADJ_CNT_REPLAY,
+    ADJ_CNT_NAN,
+    ADJ_FIRST_REPLAY,
+    ADJ_FIRST_NAN,
+    ADJ_CNT_N
+};
 
 struct AdjArgs {
     const float *state;   // [nsteps + 1][STATE_FIELDS][N]: slot k the state before step k
     int nsteps;
+    int step0;            // number of step 0 in the rollout
     const float *planes;  // the batch's planes (scale, mass, moi)
     int64_t N;
     const int *offsets;
@@ -267,7 +278,22 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
             const V3 p = add(Lb.get3(F_PX, i), mul(vi, dt));
             bad |= !veq(vi, Nx.get3(3, i)) || !veq(wi, Nx.get3(6, i)) || !veq(p, Nx.get3(0, i));
         }
-        if (__syncthreads_count(bad) && tid == 0) atomicAdd(&a.cnt[ADJ_CNT_REPLAY], 1ull);
+        if (__syncthreads_count(bad)) {  // uniform; the call then fails
+            // a NaN on both sides is no difference, though no comparison says so
+            int differs = 0;
+            for (int i = tid; i < n; i += BLOCK) {
+                for (int f = F_PX; f < F_AX; ++f) {  // P, V, W
+                    const float x = f < F_VX ? Lb.at(f, i) + Lb.at(F_VX + f, i) * dt : Lb.at(f, i), y = Nx.at(f, i);
+                    differs |= !(x == y || (x != x && y != y));
+                }
+            }
+            differs = __syncthreads_count(differs);
+            const unsigned long long at = ((unsigned long long)(a.step0 + step) << 32) | (unsigned)w;
+            if (tid == 0) {
+                atomicAdd(&a.cnt[differs ? ADJ_CNT_REPLAY : ADJ_CNT_NAN], 1ull);
+                atomicMax(&a.cnt[differs ? ADJ_FIRST_REPLAY : ADJ_FIRST_NAN], ~at);
+            }
+        }
 
         // reverse SolveConstraints, latest round first
         ContactReplay rp;
@@ -677,11 +703,12 @@ int nans_adjoint(nans_ctx *ctx, const nans_adjoint_io *io)
     a.cnt = T->cnt;
     NANS_TRY(setup_floor(ctx, s));
     int rc = NANS_OK;
-    auto reverse = [&](int nsteps) {
+    auto reverse = [&](int first, int nsteps) {
+        a.step0 = first;
         a.nsteps = nsteps;
         return W->nmax <= 64 ? adjoint_launch<64, false>(ctx, a, s) : adjoint_launch<256, false>(ctx, a, s);
     };
-    if (whole) rc = reverse(T->steps);
+    if (whole) rc = reverse(0, T->steps);
     for (int j = whole ? -1 : T->ncp - 1; j >= 0 && rc == NANS_OK; --j) {
         const int t0 = j * T->every;
         const int len = std::min(T->every, T->steps - t0);
@@ -690,7 +717,7 @@ int nans_adjoint(nans_ctx *ctx, const nans_adjoint_io *io)
         if (rc == NANS_OK)
             rc = batched_run_recorded(ctx, len, s,
                                       BatchRecord{T->seg, T->seg_rec, T->total, T->rec_off, T->seg_cnt, T->rec_cap});
-        if (rc == NANS_OK) rc = reverse(len);
+        if (rc == NANS_OK) rc = reverse(t0, len);
     }
     // back to the state after the rollout, and the statistics before this call
     if (rc == NANS_OK) rc = load_state(W, T->last, s);
@@ -701,9 +728,15 @@ int nans_adjoint(nans_ctx *ctx, const nans_adjoint_io *io)
     NANS_HIP(hipMemcpy(c, T->cnt, sizeof(c), hipMemcpyDeviceToHost));
     NANS_REQUIRE(c[ADJ_CNT_OVERFLOW] == 0, NANS_ERR_CAPACITY,
                  "a world had more contacts in one step than the adjoint keeps (16 per body + 64)");
+    auto step_of = [&](int k) { return (int)(~c[k] >> 32); };
+    auto world_of = [&](int k) { return (int)(unsigned)~c[k]; };
     NANS_REQUIRE(c[ADJ_CNT_REPLAY] == 0, NANS_ERR_STATE,
-                 "the adjoint's replay of a step did not reproduce the rollout (%llu world-steps)",
-                 (unsigned long long)c[ADJ_CNT_REPLAY]);
+                 "the adjoint's replay of a step did not reproduce the rollout (%llu world-steps, the first: step %d "
+                 "of world %d)",
+                 c[ADJ_CNT_REPLAY], step_of(ADJ_FIRST_REPLAY), world_of(ADJ_FIRST_REPLAY));
+    NANS_REQUIRE(c[ADJ_CNT_NAN] == 0, NANS_ERR_STATE,
+                 "the rollout's state is not a number in %llu world-steps, from step %d of world %d on: no gradient",
+                 c[ADJ_CNT_NAN], step_of(ADJ_FIRST_NAN), world_of(ADJ_FIRST_NAN));
     // outputs
     std::vector<float> h((size_t)12 * N);
     NANS_HIP(hipMemcpy(h.data(), T->adj, sizeof(float) * h.size(), hipMemcpyDeviceToHost));
