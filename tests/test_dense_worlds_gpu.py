@@ -40,14 +40,14 @@ def _mixed(nbox, nsph, seed):
 
 # Bytes of a contact's terms (35 words), and an upper bound of the terms a step has room
 # for: all of a CU's LDS in the plain step; in the batched one the radii and polytopes (12 KB
-# a wave at most), and two fifths of a contact record per candidate in scratch.
+# a wave at most), and a contact record (20 words) per candidate in scratch.
 TERMS = 140
 
 
 def _room(path, n, npairs, threads):
     if path == "plain":
         return 160 * 1024 // TERMS
-    return (4 * n + 12 * 1024 * max(threads, 64) // 64) // TERMS + 2 * npairs // 5
+    return (4 * n + 12 * 1024 * max(threads, 64) // 64) // TERMS + 4 * npairs // 7
 
 
 @pytest.mark.parametrize("warm", [False, True])
