@@ -320,8 +320,9 @@ int nans_reset_stats(nans_ctx *ctx);
  * nans_rollout advances every world by nsteps batched steps from the current
  * state, as nans_step_batched does, and keeps the state (pos, vel, angvel,
  * angles, force, torque) and the contacts of every step on the device while that
- * takes at most 8 GiB and a quarter of the free memory, else the state every
- * checkpoint_every steps (also where the batch records its contacts).
+ * takes at most 8 GiB (nans_set_rollout_memory) and a quarter of the free memory,
+ * else the state every checkpoint_every steps (also where the batch records its
+ * contacts).
  *
  * nans_adjoint returns the gradient of a loss L(final state) with respect to the
  * initial state and the per-body mass and moment of inertia and the per-world
@@ -331,12 +332,18 @@ int nans_reset_stats(nans_ctx *ctx);
  * (code/nans.cpp:1331-1349); the GJK/EPA outcome -- which pairs touch, in which
  * order, with which normal and lever arms PointA - PosA, PointB - PosB -- is held
  * fixed at the rollout's.  Where only checkpoints were kept, the segments between
- * them are recomputed on the device.  The mass gradient counts mass only: when the moment of inertia is a
- * function of the mass, add dl_moi * d(moi)/d(mass).  The batch is left at the
- * rollout's final state.  Arrays are host memory: vectors [3][N] planes, dl_mass
+ * them are recomputed on the device.  The mass gradient counts mass only: when the
+ * moment of inertia is a function of the mass, add dl_moi * d(moi)/d(mass).  The
+ * batch is left at the rollout's final state.  Arrays are host memory: vectors [3][N] planes, dl_mass
  * and dl_moi [N], dl_friction and dl_restitution [nworlds]; NULL inputs count as
  * zero, NULL outputs are skipped.  At most 128 impulse iterations. */
 int nans_rollout(nans_ctx *ctx, int32_t nsteps, int32_t checkpoint_every);
+
+/* Most device memory that later rollouts of the context keep for every step's state
+ * and contacts; 0 keeps checkpoints only, negative restores the default of 8 GiB.
+ * Gradients are the same either way.  A batch that holds more gives it back with its
+ * next rollout. */
+int nans_set_rollout_memory(nans_ctx *ctx, int64_t max_bytes);
 
 typedef struct nans_adjoint_io {
     const float *dl_pos, *dl_vel, *dl_angvel, *dl_angles;  /* in: dL/d(final state) */

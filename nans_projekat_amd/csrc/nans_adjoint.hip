@@ -424,13 +424,12 @@ struct AdjointTape {
 };
 
 // The dense tape: a rollout keeps every step's state and contacts while that takes at
-// most ADJ_TAPE_BYTES and a quarter of the free memory, so that the adjoint need not
+// most the context's tape_bytes and a quarter of the free memory, so that the adjoint need not
 // step the batch a second time (1024 worlds of 16 bodies, 240 steps, 1.5 GB: rollout
 // and gradient 43 -> 21.7 ms; 24 of 9, 50 steps: 6.2 -> 3.5).  Room for
 // ADJ_TAPE_CONTACTS contacts per body and step; a rollout with more is differentiated
 // through its checkpoints, as is one past the bounds, and the next one gets the room
 // it needed.
-constexpr size_t ADJ_TAPE_BYTES = (size_t)8 << 30;
 constexpr int ADJ_TAPE_CONTACTS = 4;
 
 static void free_dense(AdjointTape *T)
@@ -453,19 +452,20 @@ static int need_states(AdjointTape *T, size_t slots, size_t slot_floats)
 }
 
 // Room for a dense tape of nsteps steps; false where it does not fit.
-static bool dense_prepare(nans_worlds *W, AdjointTape *T, int nsteps)
+static bool dense_prepare(nans_worlds *W, AdjointTape *T, int nsteps, int64_t limit)
 {
     const size_t slot = (size_t)STATE_FIELDS * W->N, lists = (size_t)W->nworlds * nsteps;
     const size_t recs = std::max((size_t)ADJ_TAPE_CONTACTS * W->N * nsteps, T->rec_need);
     if (recs == 0 || recs > INT_MAX) return false;
-    if (T->rec_steps == nsteps && T->nslots == (size_t)nsteps + 1) return true;
     const size_t bytes = sizeof(float) * slot * (nsteps + 1) + sizeof(ContactRec) * recs + 2 * sizeof(int) * lists;
+    if (bytes > (size_t)limit) return false;
+    if (T->rec_steps == nsteps && T->nslots == (size_t)nsteps + 1) return true;
     free_dense(T);
     wfree(T->states);
     T->states = nullptr;
     T->nslots = 0;
     size_t avail = 0, all = 0;
-    if (hipMemGetInfo(&avail, &all) != hipSuccess || bytes > std::min(ADJ_TAPE_BYTES, avail / 4)) return false;
+    if (hipMemGetInfo(&avail, &all) != hipSuccess || bytes > avail / 4) return false;
     if (dmalloc(&T->rec, recs) || dmalloc(&T->rec_start, lists) || dmalloc(&T->rec_cnt, lists) ||
         need_states(T, (size_t)nsteps + 1, slot)) {
         (void)hipGetLastError();  // an allocation refused is no error of the rollout
@@ -550,6 +550,13 @@ using namespace nans;
 
 extern "C" {
 
+int nans_set_rollout_memory(nans_ctx *ctx, int64_t max_bytes)
+{
+    NANS_REQUIRE(ctx, NANS_ERR_INVALID, "ctx is NULL");
+    ctx->tape_bytes = max_bytes < 0 ? ADJ_TAPE_BYTES : max_bytes;
+    return NANS_OK;
+}
+
 int nans_rollout(nans_ctx *ctx, int32_t nsteps, int32_t checkpoint_every)
 {
     NANS_REQUIRE(ctx && ctx->worlds, NANS_ERR_STATE, "no worlds uploaded");
@@ -577,7 +584,7 @@ int nans_rollout(nans_ctx *ctx, int32_t nsteps, int32_t checkpoint_every)
     T->steps = 0;
     T->ncp = ncp;
     // (a batch that records its contacts keeps them in its own buffers)
-    T->dense = !W->record && dense_prepare(W, T, nsteps);
+    T->dense = !W->record && dense_prepare(W, T, nsteps, ctx->tape_bytes);
     if (!T->dense) {
         free_dense(T);
         NANS_TRY(need_states(T, ncp, slot));

@@ -260,6 +260,7 @@ int nans_create(nans_ctx **out, const nans_params *p)
     c->np_qidx = nullptr;
     c->np_qsim = nullptr;
     c->na_scratch = nullptr;
+    c->tape_bytes = ADJ_TAPE_BYTES;
     rc = noalloc_scratch_init(q.device, &c->na_scratch);
     if (rc) {
         delete c;

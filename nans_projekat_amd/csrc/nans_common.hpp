@@ -58,6 +58,9 @@ namespace nans {
 int worlds_release(nans_ctx *ctx);  // frees the world batch of a context
 }
 
+// Bound of a rollout's tape of every step where the caller sets none.
+constexpr int64_t ADJ_TAPE_BYTES = (int64_t)8 << 30;
+
 struct nans_ctx {
     nans_params p;
     hipStream_t stream;          // stream the calls are ordered on
@@ -70,4 +73,5 @@ struct nans_ctx {
     int broadphase;                  // NANS_BROADPHASE_* of the plain step
     int orientation;                 // NANS_ORIENT_* of both steps
     int warm;                        // opt-in warm start of the plain and batched steps
+    int64_t tape_bytes;              // most that a rollout's tape of every step may take
 };

@@ -354,6 +354,11 @@ class Context:
         self._sync_stream()
         check(self.lib.nans_rollout(self.h, int(nsteps), int(checkpoint_every)))
 
+    def set_rollout_memory(self, max_bytes: int = -1) -> None:
+        """Most device memory that later rollouts keep for every step's state and contacts
+        (0: checkpoints only; -1: the default, 8 GiB).  Gradients are the same either way."""
+        check(self.lib.nans_set_rollout_memory(self.h, ctypes.c_int64(int(max_bytes))))
+
     def adjoint(self, dl_pos=None, dl_vel=None, dl_angvel=None, dl_angles=None) -> dict:
         """Gradient of a loss of the final state through the last rollout(), given
         dL/d(final pos, vel, angvel, angles) as [N][3] arrays (None = zero).
