@@ -1,4 +1,5 @@
-"""What a rollout keeps on the device: the caller's bound of the tape of every step."""
+"""What a rollout keeps on the device: the caller's bound of the tape of every step, and
+the tape of a longer rollout serving a shorter one."""
 import numpy as np
 import pytest
 import torch
@@ -48,4 +49,45 @@ def test_caller_bounds_the_tape():
     for g in got[1:]:
         for k, v in got[0].items():
             np.testing.assert_array_equal(g[k], v, err_msg=k)
+    ctx.close()
+
+
+def test_a_shorter_rollout_fits_the_tape():
+    """After 160 steps' tape (245 MiB), rollouts of 100 and 41 steps allocate and free
+    nothing; one of 16 takes a tape of its own (25 MiB).  Each gives the gradient that it
+    gives on a context of its own, and so does 160 again."""
+    sc, ctx = _batch()
+    want = {}
+    for n in (16, 41, 100, 160):
+        _, own = _batch()
+        want[n] = _gradient(sc, own, n, 7)
+        own.close()
+    _gradient(sc, ctx, 160, 7)
+    before = _free()
+    for n, lo, hi in ((160, -1, 1), (100, -1, 1), (41, -1, 1), (160, -1, 1), (16, 200, 240), (160, -1, 1)):
+        got = _gradient(sc, ctx, n, 7)
+        assert lo < (_free() - before) / MIB < hi, (n, _free() - before)
+        for k, v in want[n].items():
+            np.testing.assert_array_equal(got[k], v, err_msg="%d %s" % (n, k))
+    ctx.close()
+
+
+def test_refusal_keeps_the_checkpoints():
+    """A rollout that may not keep a tape uses the buffer of the one before it, whether that
+    was refused too or had a tape, and gradients do not depend on it."""
+    sc, ctx = _batch(64)
+    _, own = _batch(64)
+    want = [_gradient(sc, own, 24, 5), _gradient(sc, own, 31, 5)]
+    own.close()
+    ctx.set_rollout_memory(0)
+    for n, i in ((24, 0), (24, 0), (31, 1), (24, 0)):
+        got = _gradient(sc, ctx, n, 5)
+        for k, v in want[i].items():
+            np.testing.assert_array_equal(got[k], v, err_msg="%d %s" % (n, k))
+    ctx.set_rollout_memory(-1)
+    for limit in (-1, 0, -1):
+        ctx.set_rollout_memory(limit)
+        got = _gradient(sc, ctx, 24, 5)
+        for k, v in want[0].items():
+            np.testing.assert_array_equal(got[k], v, err_msg=k)
     ctx.close()
