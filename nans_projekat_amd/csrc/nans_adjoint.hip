@@ -610,6 +610,9 @@ int nans_rollout(nans_ctx *ctx, int32_t nsteps, int32_t checkpoint_every)
         BatchRecord r{T->states, T->rec, 0, nullptr, T->rec_cnt, nullptr, T->pos, T->rec_start, T->rec_total};
         NANS_TRY(batched_run_recorded(ctx, nsteps, s, r));
         NANS_HIP(hipMemcpyAsync(&used, T->pos, sizeof(used), hipMemcpyDeviceToHost, s));
+        // nans_batched_timing answers after any batched launch; without an
+        // nans_step_batched call before, as after the last checkpoint's launch
+        if (W->timed_steps == 0) W->timed_steps = nsteps - (ncp - 1) * checkpoint_every;
     } else {
         const int block = batched_block(ctx);
         for (int j = 0; j < ncp; ++j) {

@@ -91,3 +91,20 @@ def test_refusal_keeps_the_checkpoints():
         for k, v in want[0].items():
             np.testing.assert_array_equal(got[k], v, err_msg=k)
     ctx.close()
+
+
+@pytest.mark.parametrize("limit", [-1, 0])
+def test_batched_timing_after_a_rollout(limit):
+    """nans_batched_timing names the launch shape after a rollout as after a step, with a
+    tape and with checkpoints; before either it refuses."""
+    sc, ctx = _batch(4)
+    ctx.set_rollout_memory(limit)
+    with pytest.raises(runtime.NansError):
+        ctx.batched_timing()
+    ctx.rollout(7, 3)
+    t = ctx.batched_timing()
+    assert t["workgroups"] > 0 and t["threads_per_world"] == 128 and t["steps"] == 1 and t["elapsed_ms"] == 0.0
+    ctx.step_batched(5)
+    t = ctx.batched_timing()
+    assert t["steps"] == 5 and t["elapsed_ms"] > 0.0
+    ctx.close()
