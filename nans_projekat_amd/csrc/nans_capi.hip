@@ -350,7 +350,9 @@ static int narrow_launch(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, con
         int shift = 0;  // of a share
         while (2 << shift <= NP_SHARE && (2 << shift) * 4 * waves <= n) ++shift;
         const int64_t shares = (n + (1 << shift) - 1) >> shift;
-        const unsigned grid = (unsigned)std::min<int64_t>((shares + 3) / 4, waves / 4);
+        unsigned grid = (unsigned)std::min<int64_t>((shares + 3) / 4, waves / 4);
+        // as many workgroups to every group: 200 pairs on 50 left some groups a claim short
+        if (grid > NP_GROUPS) grid = (grid + NP_GROUPS - 1) / NP_GROUPS * NP_GROUPS;
         const NarrowParams np = narrow_params(ctx->p);
         if (ctx->p.fp64_islands)
             k_narrowphase<true><<<grid, 256, 0, s>>>(n, shift, ia, ib, np, o, cnt, qidx, qsim);
