@@ -111,7 +111,8 @@ constexpr int NP_WAVES_PER_CU = 12;
 // alike within 5 %).
 constexpr int NP_GROUPS = 32;
 constexpr int NP_CNT_STRIDE = 16;
-constexpr int NP_CNT_WORDS = NP_CNT_STRIDE * (1 + NP_GROUPS);  // [0]: the overflow count
+constexpr int NP_CNT_WORDS = NP_CNT_STRIDE * NP_GROUPS;
+constexpr int NP_CNT_OVERFLOW = 1;  // the word of the overflow count, beside the first counter
 // A wave that has seen this many pairs in a row miss takes twice as many with its next
 // claim, up to 64, until a pair hits: one share fills few lanes of GJK, and only hits
 // make a share long (all miss, 200k / 1M: 60 / 101 -> 47 / 69 us; at 32 in a row 52 / 69;
@@ -138,13 +139,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NP_WAVES_PE
     int64_t first = (int64_t)(4 * ((int)blockIdx.x / groups) + wv) << shift;  // a wave's first share is its own
     while (first < mine) {
         const int count = (int)min((int64_t)take, mine - first);
-        PairSrc src{a, b, first, n, groups, g, shift, o, &cnt[0], sim + before + first};
+        PairSrc src{a, b, first, n, groups, g, shift, o, &cnt[NP_CNT_OVERFLOW], sim + before + first};
         run = narrow_wave<ISL>(src, count, p, lds[wv], list + before + first) ? 0 : run + count;
         if (started >= mine) break;  // the first shares were all
         take = run >= NP_RUN ? min(64, 2 * take) : 1 << shift;
         unsigned long long c = 0;
         wave_sync();  // the wave meets on both sides of the claim
-        if (lane_id() == 0) c = atomicAdd(&cnt[NP_CNT_STRIDE * (1 + g)], (unsigned long long)take);
+        if (lane_id() == 0) c = atomicAdd(&cnt[NP_CNT_STRIDE * g], (unsigned long long)take);
         wave_sync();
         first = started + (int64_t)(((unsigned long long)__builtin_amdgcn_readfirstlane((int)(c >> 32)) << 32) |
                                     (unsigned)__builtin_amdgcn_readfirstlane((int)c));
@@ -361,7 +362,7 @@ static int narrow_launch(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, con
         NANS_HIP(hipGetLastError());
     }
     unsigned long long ov = 0;
-    NANS_HIP(hipMemcpyAsync(&ov, cnt, sizeof(ov), hipMemcpyDeviceToHost, s));
+    NANS_HIP(hipMemcpyAsync(&ov, cnt + NP_CNT_OVERFLOW, sizeof(ov), hipMemcpyDeviceToHost, s));
     NANS_HIP(hipStreamSynchronize(s));
     if (n_overflow) *n_overflow = (int64_t)ov;
     return NANS_OK;
