@@ -3,7 +3,7 @@
 
 Headline: config 3 -- 4096 independent worlds of 8..256 bodies (log-uniform),
 box stacks hit by 1-4 spheres, dt = 1/120, 10 impulse iterations -- advanced
-by the batched step (one persistent launch per step, replayed from a hipGraph).
+by the batched step (one persistent launch per call, per 256 steps of a longer one).
 A "step" is one step of all 4096 worlds; value = world-body-steps/s over the K
 timed steps, with the state resident in HBM.  The timed region starts from
 the scene's initial state (it is restored after the warmup), so K = 240 is
@@ -21,10 +21,10 @@ Also reported on the same line:
   opt_in_modes    the quaternion orientation (config 3, batched) and the warm start
                   (config 5, plain; config 3, batched) beside the reference's modes
                   on the same steps;
-  roofline        the batched step kernel: algorithmic FP32 flops per launch
+  roofline        the batched step kernel: algorithmic FP32 flops of the timed steps
                   (event counts frozen in tests/golden/work_counts.json times the
-                  per-event weights below) over its average launch time, timed
-                  with HIP events on the stream it runs on;
+                  per-event weights below) over its launch time, timed with HIP
+                  events on the stream it runs on;
   cpu_baseline    the CPU oracle (binary32 restatement of the reference step,
                   brute-force all pairs as the reference does) on a bounded
                   sample of config-3 worlds, one process per core.
@@ -69,6 +69,7 @@ FLOP_WEIGHTS = {
     "constraints": 400,      # Jacobians, effective masses, impulse application
     "solver_iterations": 14, # one accumulate/clamp iteration
 }
+BATCH_LAUNCH_STEPS = 256  # steps of one launch of the batched kernel at most
 STATE_BYTES_PER_BODY_STEP = 164  # read P,V,W,A,S,m,I,F,T (92 B), write P,V,W,A and cleared F,T (72 B)
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "k_batched_step_config3.md")
 
@@ -78,14 +79,14 @@ NP_BYTES_PER_PAIR = 108      # 2 shapes x 44 B in (type, centre, quaternion, hal
 NP_ABI_BYTES_PER_PAIR = 144  # this ABI: 88 B in, 56 B out (flags, status, normal, depth, both points)
 
 
-def measured_traffic(path=TRAFFIC_PROFILE):
-    """HBM bytes per launch of a kernel: rocprofv3 FETCH_SIZE plus WRITE_SIZE,
-    each scaled by what the counter reads for a 1 GiB device copy (the profile
-    file records the commands and the factors)."""
+def measured_traffic(path, per):
+    """HBM bytes of a kernel per launch or per step: rocprofv3 FETCH_SIZE plus
+    WRITE_SIZE, each scaled by what the counter reads for a 1 GiB device copy (the
+    profile file records the commands and the factors)."""
     if not os.path.exists(path):
         return None
     with open(path) as f:
-        m = re.search(r"^traffic_bytes_per_launch: (\d+)$", f.read(), re.M)
+        m = re.search(r"^traffic_bytes_per_%s: (\d+)$" % per, f.read(), re.M)
     return int(m.group(1)) if m else None
 
 
@@ -293,7 +294,7 @@ def narrowphase_leg(args, work):
         fl = algorithmic_flops(c2) / c2["n_pairs"] * n
         tf = fl / (np_ms * 1e-3) / 1e12
         gb = NP_BYTES_PER_PAIR * n / (np_ms * 1e-3) / 1e9
-        tr = measured_traffic(NP_TRAFFIC_PROFILE)
+        tr = measured_traffic(NP_TRAFFIC_PROFILE, "launch")
         res["roofline"] = {
             "bound": "valu", "achieved": round(tf, 4), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
             "frac": round(tf / PEAK_FP32_TFLOPS, 5), "traffic": tr,
@@ -354,7 +355,7 @@ def differentiable_leg(args):
     dctx.upload(dif)
     dl = np.full((dif.nbodies, 3), 1e-3, np.float32)
     dctx.rollout(8, 4)
-    dctx.adjoint(dl_pos=dl)  # warm-up: graph capture, scratch allocation
+    dctx.adjoint(dl_pos=dl)  # warm-up: scratch allocation
     dctx.set_state(dif)
     torch.cuda.synchronize()
     d0 = time.perf_counter()
@@ -455,16 +456,19 @@ def main():
         flops, exact, cand = window_flops(work, args.steps)
         tflops = flops / args.steps / (kernel_ms * 1e-3) / 1e12
         gbs = STATE_BYTES_PER_BODY_STEP * sc.nbodies / (kernel_ms * 1e-3) / 1e9
-        traffic = measured_traffic()
+        traffic = measured_traffic(TRAFFIC_PROFILE, "step")
+        launches = -(-args.steps // BATCH_LAUNCH_STEPS)
         roof = {"bound": "valu", "achieved": round(tflops, 4), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                 "frac": round(tflops / PEAK_FP32_TFLOPS, 5), "traffic": traffic,
-                "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE per launch (calibrated on a device copy), "
+                "traffic_source": "rocprofv3 FETCH_SIZE + WRITE_SIZE per step (calibrated on a device copy), "
                                   "from %s, not measured in this run" % os.path.relpath(TRAFFIC_PROFILE, ROOT)
                                   if traffic else None,
                 "kernel": "k_batched_step",
                 "compute": "vector FP32 (VALU): nothing on the path is a dense contraction and the kernels issue "
                            "no MFMA; peak = MI355X FP32 vector",
-                "flops_per_launch": round(flops / args.steps), "avg_launch_ms": round(kernel_ms, 5),
+                "flops_per_step": round(flops / args.steps), "kernel_ms_per_step": round(kernel_ms, 5),
+                "launches": launches, "flops_per_launch": round(flops / launches),
+                "avg_launch_ms": round(timing["elapsed_ms"] / launches, 5),
                 "flops_window": "oracle event counts of steps [0, %d) of config 3 (the timed steps), times the "
                                 "per-event weights" % args.steps if exact else
                                 "steps beyond the frozen 240: the 240-step average per step",

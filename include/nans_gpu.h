@@ -135,12 +135,12 @@ int nans_narrowphase(nans_ctx *ctx, int64_t n, const nans_shapes_soa *a, const n
                      const nans_narrow_out *out, int64_t *n_overflow);
 
 /* nans_narrowphase without any device allocation.  No counterpart in the
- * reference: it is for callers that cannot allocate device memory (code under
- * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
+ * reference: it is for callers that cannot allocate device memory (tight
+ * serving loops, harnesses that forbid hipMalloc).
  * Same arguments, results and errors as nans_narrowphase, except that at most
  * NANS_NARROWPHASE_NOALLOC_MAX_PAIRS pairs are accepted per call (more:
- * NANS_ERR_CAPACITY; split the call).  Its EPA queue lives in a static device
- * array of 26 MiB per device, held until the process ends and shared by every
+ * NANS_ERR_CAPACITY; split the call).  Its hit list lives in a static device
+ * array of 27 MiB per device, held until the process ends and shared by every
  * call on that device: calls that overlap on one device (several threads or
  * streams at once) race on it. */
 #define NANS_NARROWPHASE_NOALLOC_MAX_PAIRS 262144

@@ -1421,10 +1421,12 @@ static size_t batch_lds_bytes(int nmax, const WaveSplit &sp, int block)
 }
 
 // Default bound of the worlds run one per wave: none.  A world on one wave takes
-// 1.5x (8-15 bodies) to 2.9x (32-63 bodies) as long as on a 256-thread
-// workgroup, so the wave phase, which runs last, lengthens the step's tail more
-// than it saves (config 3 on the MI355X: 1.93 ms per step at bound 0, 1.92 at
-// 16, 2.12 at 64); the autotuner tries the bounds per batch.
+// longer than on a 256-thread workgroup, and the wave phase runs last, so it pays
+// only where a launch has many steps and worlds to even out (ms a step at bounds 0,
+// 16, 32, 64: 4096 worlds of 8-256 bodies, 20 steps a launch 0.833, 0.826, 0.822,
+// 0.849, 240 steps 0.793, 0.771, 0.736, 0.735; 2048 worlds, 60 steps 0.429, 0.438,
+// 0.445, 0.474; 1024 and 512 alike within 2 %); the autotuner tries the bounds per
+// batch.
 constexpr int WAVE_WORLD_BODIES = 0;
 
 // The wave-world bound at a workgroup size: none at one wave per workgroup.
@@ -1723,7 +1725,7 @@ int nans_upload_worlds(nans_ctx *ctx, int32_t nworlds, const int32_t *world_offs
 // Batches of up to this many bodies pass their state through one staging copy (a copy's
 // fixed cost, some 10 us, counts); larger ones field by field, without staging
 // (set_state, 60 steps and download of 295k bodies: 67.8 -> 55.2 ms, most of it the
-// quaternions no longer made; one step and a download of 28 bodies 158 -> 149 us).
+// quaternions no longer made).
 constexpr int64_t STAGE_BODIES = 8192;
 
 int nans_download_state(nans_ctx *ctx, nans_bodies_soa *b)
